@@ -34,8 +34,8 @@ DEFAULT_OUT = os.path.join(HERE, "schedule.json")
 
 # candidate values per field, in the order they are tuned (the default first)
 CANDIDATES = {
-    "kmax_big": [384, 192, 256, 512, 768, 1024],
-    "kmax_small": [96, 48, 64, 128, 192],
+    "kmax_big": [0, 384, 192, 256, 512, 768, 1024],
+    "kmax_small": [0, 96, 48, 64, 128, 192],
     "march_zn": [0, 8, 16],
     "big_halo": [2048, 1024, 4096, 8192],
     "wave_halo": [512, 256, 1024],

@@ -635,4 +635,33 @@ AHF_HD int ahf_fold_T_in(int64_t K, int64_t R, int neg)
   return neg ? (T <= -lo && T >= -hi) : (T >= lo && T <= hi);
 }
 
+/*
+ * One contribution of a whole block of them (the heavy kernels' block sum):
+ * the step r of K for a value in the binade whose ulp is 1/scale, in FP64
+ * alone.  x = c/ulp (exact: a power of two); y = x + 1.5*2^23 lies in
+ * [2^23, 2^24) for |x| < 2^22, where doubles are 2^-29 apart, as AHF's
+ * double sum K + x is inside the binade, and 1.5*2^23 - K is an even number
+ * of those steps: y rounds as that sum does.  r = y rounded to an integer,
+ * less 1.5*2^23, unless y is half way between two (the parity of K would
+ * decide).  Returns 1 when r is the step whatever K is, as long as the step
+ * ends inside the binade and not on its edge; 0 for a tie, a large
+ * contribution or a NaN.
+ */
+AHF_HD int ahf_fold_step(double c, double scale, int32_t *r)
+{
+  const double M = 12582912.0; /* 1.5 * 2^23 */
+  const double x = c * scale, y = x + M, n = rint(y);
+  const int ok = fabs(x) < 4194304.0 && fabs(y - n) != 0.5;
+  *r = ok ? (int32_t)(n - M) : 0;
+  return ok;
+}
+/* K (a running value in its binade) moved by the sum S of the steps of a
+ * block of contributions none of which is negative: 1 when no step of the
+ * block leaves the binade, whatever their order */
+AHF_HD int ahf_fold_block_in(int64_t K, int64_t S)
+{
+  const int64_t E = K + S;
+  return K > 0 ? E < ((int64_t)1 << 24) : E < -((int64_t)1 << 23);
+}
+
 #endif /* AHF_AMR_CORE_H */

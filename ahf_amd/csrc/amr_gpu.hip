@@ -9,7 +9,7 @@
  *   k_pmask        presence mask of every node (get_TSCnodes rules)
  *   k_prep         particle-node separations of every bucket entry
  *   k_gather_light exact-order TSC density, one lane per node (assign_npart)
- *   k_gather_heavy the same, one wavefront per node with many contributions
+ *   k_gather_heavy the same, nodes with many contributions, by wavefronts
  *   k_flags        interior + refinement criterion (test_node)
  *   k_refine_rows  ref_pquad/ref_cquad/ref_nquad block tests and run state
  *                  machine, one thread per level row
@@ -30,6 +30,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/ahf_gpu.h"
@@ -158,18 +159,21 @@ __global__ void k_pmask(level_view v, uint32_t *__restrict__ pmask, uint8_t *__r
 }
 
 /* weight record of every bucket entry (entries [0, *n)): its particle's
- * TSC weights against the entry's own node */
+ * TSC weights against the entry's own node; and its position record, which
+ * the heavy targets and the relinking read */
 __global__ void k_prep(level_view v, const int64_t *__restrict__ n_ptr, int64_t n_max,
                        const uint32_t *__restrict__ pnode, const uint32_t *__restrict__ plist,
                        const float *__restrict__ px, const float *__restrict__ py, const float *__restrict__ pz,
-                       double m2pd, ahf_w9 *__restrict__ W)
+                       double m2pd, ahf_w9 *__restrict__ W, ahf_q4 *__restrict__ qp)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n_max || q >= *n_ptr) return;
   const uint32_t p = plist[q];
+  const ahf_q4 e = {px[p], py[p], pz[p], 0.0f};
   ahf_w9 w;
-  ahf_entry_weights(&v, (int64_t)pnode[q], px[p], py[p], pz[p], m2pd, &w);
+  ahf_entry_weights(&v, (int64_t)pnode[q], e.x, e.y, e.z, m2pd, &w);
   W[q] = w;
+  qp[q] = e;
 }
 
 /* position record of every bucket entry (entries [0, *n)), for the
@@ -250,11 +254,16 @@ __device__ __forceinline__ int rot_offset(int i, int r)
   return (v >= 3 ? v - 3 : v) - 1;
 }
 
-/* the three weights of record q for a source at offset (ex,ey,ez) */
-__device__ __forceinline__ double w9_contrib(const ahf_w9 *__restrict__ W, uint32_t q, int iz, int iy, int ix)
+/* a target with more contributions than this is folded by a workgroup
+ * (heavy_targets): fewer fill its wavefronts only once */
+#define AHF_HUGE 2048
+/* target n of `total` contributions for the heavy kernels: the list's front,
+ * or its back (nn entries, one a node) for the huge ones */
+__device__ __forceinline__ void heavy_push(uint32_t *__restrict__ heavy, uint32_t *__restrict__ n_heavy, int64_t nn,
+                                           int64_t n, uint64_t total)
 {
-  const double *w = reinterpret_cast<const double *>(W + q);
-  return w[iz] * w[3 + iy] * w[6 + ix];
+  if (total > AHF_HUGE) heavy[nn - 1 - (int64_t)atomicAdd(n_heavy + 1, 1u)] = (uint32_t)n;
+  else heavy[atomicAdd(n_heavy, 1u)] = (uint32_t)n;
 }
 
 /*
@@ -348,7 +357,7 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_light(level_view v, const 
         }
       }
   if (total > kmax) {
-    heavy[atomicAdd(n_heavy, 1u)] = (uint32_t)n;
+    heavy_push(heavy, n_heavy, 8 * v.n_oct, n, total);
     return;
   }
   const uint32_t step = descending ? 0xFFFFFFFFu : 1u;
@@ -517,7 +526,7 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_src(level_view v, const ui
         if ((r.z >> ((1 - ez) * 9 + (1 - ey) * 3 + (1 - ex))) & 1u) total += r.y;
       }
   if (total > kmax) {
-    heavy[atomicAdd(n_heavy, 1u)] = (uint32_t)n;
+    heavy_push(heavy, n_heavy, 8 * v.n_oct, n, total);
     return;
   }
   const double L = (double)v.L;
@@ -560,9 +569,8 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_src(level_view v, const ui
 #define AHF_SLAB 16                          /* target tile: 16x16 nodes of one plane */
 #define AHF_SLAB_W (AHF_SLAB + 2)            /* its sources in one plane: 18x18 nodes */
 #define AHF_SLAB_N (AHF_SLAB_W * AHF_SLAB_W)
-#define AHF_SLAB_CAP_BIG 2752                /* staged entries per plane, dense levels */
-#define AHF_SLAB_CAP_SMALL 512               /* the same for about one entry per node */
-#define AHF_MARCH_CAP_SMALL 448              /* the marching walk at about one entry per node */
+#define AHF_FULL_CAP_BIG 2752                /* staged entries per plane, dense levels */
+#define AHF_FULL_CAP_SMALL 448               /* the same for about one entry per node */
 
 /* node (X,Y,Z) of a level that holds every octet: its octets are all
  * (L/2)^3 keys in (z,y,x) order */
@@ -571,6 +579,22 @@ __device__ __forceinline__ int64_t full_node(int64_t X, int64_t Y, int64_t Z, in
   const int64_t o = ((Z >> 1) * H + (Y >> 1)) * H + (X >> 1);
   return 8 * o + ((Z & 1) << 2 | (Y & 1) << 1 | (X & 1));
 }
+
+/* LDS of one workgroup of k_gather_full: bucket start and entry count of
+ * three source planes' nodes, the slot offsets and entries of the staged one
+ * (FULL: nine weights an entry, else the three separations) */
+template <int CAP, bool FULL>
+struct FullShared {
+  double cx[AHF_SLAB_W], cy[AHF_SLAB_W];
+  double e[(FULL ? 9 : 3) * CAP];
+  uint32_t start[3 * AHF_SLAB_N], cnt[3 * AHF_SLAB_N], off[AHF_SLAB_N + 1];
+  union {
+    uint32_t slab_pm[3 * AHF_SLAB_N];
+    struct {
+      uint32_t pm[AHF_SLAB_N], q[FULL ? 9 * AHF_BLOCK : 1];
+    } march;
+  };
+};
 
 /* ahf_tsc_w(s, d) for an offset d known only at run time, as
  * A + B*(C + D*s)^2 with
@@ -594,10 +618,9 @@ struct TscRt {
 };
 
 /*
- * Exact-order density of a level that holds every octet (the domain grid,
- * and any level refined everywhere), one workgroup per 16x16 tile of target
- * nodes in one z-plane, one lane per target; with faces set only the planes
- * Z = 0 and Z = L-1, whose z order wraps (the others march, k_gather_march).
+ * Exact-order density of one 16x16 tile of target nodes of the plane Z of a
+ * level that holds every octet, by one workgroup, one lane per target: for
+ * the planes Z = 0 and Z = L-1, whose z order wraps (the others march).
  *
  * All targets of the tile share Z, so they visit the three source planes in
  * the same order (ahf_axis_order of Z).  The workgroup stages one source
@@ -609,30 +632,18 @@ struct TscRt {
  * rounds ((m2pd*wz)*wy)*wx into its FP32 node value as AHF does.  Entries of
  * nodes that do not fit in the CAP staged slots are read from the position
  * records instead, with the same arithmetic.  Targets with more than kmax
- * contributions are left to k_gather_heavy_q.  Tiles are dealt so that each
- * XCD walks a contiguous run of them (consecutive planes share two source
- * planes in its L2).
+ * contributions are left to k_gather_heavy.
  */
 template <int CAP, bool W9>
-__global__ void __launch_bounds__(AHF_BLOCK) k_gather_slab(level_view v, int64_t per_xcd,
-                                                           const uint32_t *__restrict__ pmask,
-                                                           const int64_t *__restrict__ p0,
-                                                           const ahf_q4 *__restrict__ qp, int descending,
-                                                           double m2pd, uint32_t kmax, float *__restrict__ dens,
-                                                           uint32_t *__restrict__ heavy,
-                                                           uint32_t *__restrict__ n_heavy, int faces)
+__device__ __forceinline__ void gather_slab(const level_view &v, int64_t tx, int64_t ty, int64_t Z, FullShared<CAP, W9> &S,
+                                            const uint32_t *__restrict__ pmask, const int64_t *__restrict__ p0,
+                                            const ahf_q4 *__restrict__ qp, int descending, double m2pd, uint32_t kmax,
+                                            float *__restrict__ dens, uint32_t *__restrict__ heavy,
+                                            uint32_t *__restrict__ n_heavy)
 {
-  constexpr int NV = W9 ? 7 : 3; /* doubles per staged entry */
-  __shared__ uint32_t s_start[3 * AHF_SLAB_N], s_cnt[3 * AHF_SLAB_N], s_pm[3 * AHF_SLAB_N];
-  __shared__ uint32_t s_off[AHF_SLAB_N + 1];
-  __shared__ double s_cx[AHF_SLAB_W], s_cy[AHF_SLAB_W];
-  __shared__ double s_e[NV * CAP];
-  const int64_t L = v.L, H = L >> 1, T = L / AHF_SLAB;
-  const int64_t b = blockIdx.x;
-  const int64_t tile = (b % AHF_XCDS) * per_xcd + b / AHF_XCDS;
-  if (tile >= T * T * (faces ? 2 : L)) return; /* the whole workgroup */
-  const int64_t zi = tile / (T * T), ty = (tile / T) % T, tx = tile % T;
-  const int64_t Z = faces ? (zi == 0 ? 0 : L - 1) : zi;
+  uint32_t *const s_start = S.start, *const s_cnt = S.cnt, *const s_pm = S.slab_pm, *const s_off = S.off;
+  double *const s_cx = S.cx, *const s_cy = S.cy, *const s_e = S.e;
+  const int64_t L = v.L, H = L >> 1;
   const int tid = threadIdx.x, lx = tid & (AHF_SLAB - 1), ly = tid / AHF_SLAB;
   const int64_t X = tx * AHF_SLAB + lx, Y = ty * AHF_SLAB + ly;
   const double Ld = (double)L;
@@ -673,8 +684,9 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_slab(level_view v, int64_t
         if (s_cnt[u]) mask |= 1u << (k * 9 + bb * 3 + e);
       }
   const int64_t n = full_node(X, Y, Z, H);
-  const bool active = total <= kmax;
-  if (!active) heavy[atomicAdd(n_heavy, 1u)] = (uint32_t)n;
+  const bool inside = X < L && Y < L; /* the last tile of a row or column may be partial */
+  const bool active = inside && total <= kmax;
+  if (inside && !active) heavy_push(heavy, n_heavy, 8 * v.n_oct, n, total);
   const uint32_t step = descending ? 0xFFFFFFFFu : 1u;
   float d = -1.0f;
   for (int k = 0; k < 3; k++) {
@@ -762,7 +774,7 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_slab(level_view v, int64_t
   if (active) dens[n] = d;
 }
 
-/* shared state of one marching workgroup (k_gather_march) */
+/* shared state of one marching workgroup (gather_march) */
 struct MarchView {
   const uint32_t *cnt, *start, *off; /* the walked plane's slot */
   const double *e;                   /* its staged entries */
@@ -903,7 +915,7 @@ __device__ __forceinline__ PlaneSum plane_sum(const uint32_t *cnt, const uint32_
  * every octet, whose sources lie in the planes Z-1, Z, Z+1 in that order.
  * One workgroup per 16x16 column tile and run of zn target planes, one lane
  * per (x,y) column.  The workgroup marches up through the source planes,
- * staging each one in LDS once (as in k_gather_slab), and every lane folds
+ * staging each one in LDS once (as in gather_slab), and every lane folds
  * the staged plane P into its three open targets: plane P+1 (its first
  * source plane), P (its second) and P-1 (its third, after which the value
  * is final).  All three visit the plane's sources in the same order, so one
@@ -918,31 +930,22 @@ __device__ __forceinline__ PlaneSum plane_sum(const uint32_t *cnt, const uint32_
  * the sources are walked one by one with compile-time weights.
  */
 template <int CAP, bool FULL>
-__global__ void __launch_bounds__(AHF_BLOCK) k_gather_march(level_view v, int64_t per_xcd, int64_t zn,
-                                                            const uint32_t *__restrict__ pmask,
-                                                            const int64_t *__restrict__ p0,
-                                                            const ahf_q4 *__restrict__ qp, int descending,
-                                                            double m2pd, uint32_t kmax, float *__restrict__ dens,
-                                                            uint32_t *__restrict__ heavy,
-                                                            uint32_t *__restrict__ n_heavy)
+__device__ __forceinline__ void gather_march(const level_view &v, int64_t tx, int64_t ty, int64_t T, int64_t ch, int64_t zn,
+                                             FullShared<CAP, FULL> &S, const uint32_t *__restrict__ pmask,
+                                             const int64_t *__restrict__ p0, const ahf_q4 *__restrict__ qp,
+                                             int descending, double m2pd, uint32_t kmax, float *__restrict__ dens,
+                                             uint32_t *__restrict__ heavy, uint32_t *__restrict__ n_heavy)
 {
-  constexpr int NV = FULL ? 9 : 3; /* doubles per staged entry */
-  __shared__ uint32_t s_start[3 * AHF_SLAB_N], s_cnt[3 * AHF_SLAB_N], s_pm[AHF_SLAB_N];
-  __shared__ uint32_t s_off[AHF_SLAB_N + 1];
-  __shared__ double s_cx[AHF_SLAB_W], s_cy[AHF_SLAB_W];
-  __shared__ double s_e[NV * CAP];
-  __shared__ uint32_t s_q[FULL ? 9 * AHF_BLOCK : 1];
-  const int64_t L = v.L, H = L >> 1, T = L / AHF_SLAB;
-  const int64_t nch = (L - 2 + zn - 1) / zn;
-  const int64_t b = blockIdx.x;
-  const int64_t w = (b % AHF_XCDS) * per_xcd + b / AHF_XCDS;
-  if (w >= T * T * nch) return; /* the whole workgroup */
-  const int64_t ch = w / (T * T), ty = (w / T) % T, tx = w % T;
+  uint32_t *const s_start = S.start, *const s_cnt = S.cnt, *const s_pm = S.march.pm, *const s_off = S.off,
+                  *const s_q = S.march.q;
+  double *const s_cx = S.cx, *const s_cy = S.cy, *const s_e = S.e;
+  const int64_t L = v.L, H = L >> 1;
   const int64_t Z0 = 1 + ch * zn, Z1 = Z0 + zn < L - 1 ? Z0 + zn : L - 1;
   const int tid = threadIdx.x, lx = tid & (AHF_SLAB - 1), ly = tid / AHF_SLAB;
   const int64_t X = tx * AHF_SLAB + lx, Y = ty * AHF_SLAB + ly;
   const double Ld = (double)L;
   const bool face = tx == 0 || tx == T - 1 || ty == 0 || ty == T - 1;
+  const bool inside = X < L && Y < L; /* the last tile of a row or column may be partial */
   int oy[3], ox[3];
   ahf_axis_order(Y, L, oy);
   ahf_axis_order(X, L, ox);
@@ -1065,11 +1068,11 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_march(level_view v, int64_
     mn = 0;
     an = false;
     dn = -1.0f;
-    if (P + 1 >= Z0 && P + 1 < Z1) {
+    if (inside && P + 1 >= Z0 && P + 1 < Z1) {
       const uint64_t total = (uint64_t)sP.c0 + sP1.c1 + sP2.c2;
       an = total <= kmax;
       if (an) mn = (sP.m & 0x1FFu) | (sP1.m & (0x1FFu << 9)) | (sP2.m & (0x1FFu << 18));
-      else heavy[atomicAdd(n_heavy, 1u)] = (uint32_t)full_node(X, Y, P + 1, H);
+      else heavy_push(heavy, n_heavy, 8 * v.n_oct, full_node(X, Y, P + 1, H), total);
     }
     __syncthreads();
     m.cnt = cnt_p;
@@ -1109,10 +1112,12 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_march(level_view v, int64_
         const bool r0 = m0 != 0u, r1 = m1 != 0u, r2 = m2 != 0u;
         const int oy0 = oy[0], oy1 = oy[1], oy2 = oy[2];
         uint32_t ntot = 0;
+        if (r0 || r1 || r2) {
 #pragma unroll
-        for (int bb = 0; bb < 3; bb++) {
-          const int u = (ly + 1 + oy[bb]) * AHF_SLAB_W + lx;
-          ntot += s_off[u + 3] - s_off[u];
+          for (int bb = 0; bb < 3; bb++) {
+            const int u = (ly + 1 + oy[bb]) * AHF_SLAB_W + lx;
+            ntot += s_off[u + 3] - s_off[u];
+          }
         }
         /* the current row: next entry q, entries left, range [lo, hi) with
          * inner boundaries b1, b2, and the offset of its y weight */
@@ -1244,6 +1249,41 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_gather_march(level_view v, int64_
   }
 }
 
+/*
+ * Exact-order density of a level that holds every octet, L >= AHF_SLAB, in
+ * one launch: workgroups [0, nface) take the tiles of the two face planes
+ * Z = 0 and L-1 (gather_slab), which would otherwise follow the march alone
+ * on the chip (0.29 ms of a 128^3 level's 0.60), the others the column tiles
+ * and runs of zn planes between them (gather_march).  Dealt so that each XCD
+ * walks a contiguous run of either kind (per_f and per_m workgroups an XCD).
+ */
+template <int CAP, bool FULL>
+__global__ void __launch_bounds__(AHF_BLOCK) k_gather_full(level_view v, int64_t per_f, int64_t per_m, int64_t zn,
+                                                           const uint32_t *__restrict__ pmask,
+                                                           const int64_t *__restrict__ p0,
+                                                           const ahf_q4 *__restrict__ qp, int descending,
+                                                           double m2pd, uint32_t kmax, float *__restrict__ dens,
+                                                           uint32_t *__restrict__ heavy,
+                                                           uint32_t *__restrict__ n_heavy)
+{
+  __shared__ FullShared<CAP, FULL> S;
+  const int64_t L = v.L, T = (L + AHF_SLAB - 1) / AHF_SLAB;
+  const int64_t nch = (L - 2 + zn - 1) / zn;
+  int64_t b = blockIdx.x;
+  if (b < AHF_XCDS * per_f) {
+    const int64_t w = (b % AHF_XCDS) * per_f + b / AHF_XCDS;
+    if (w >= 2 * T * T) return; /* the whole workgroup */
+    gather_slab<CAP, FULL>(v, w % T, (w / T) % T, w / (T * T) == 0 ? 0 : L - 1, S, pmask, p0, qp, descending, m2pd, kmax,
+                           dens, heavy, n_heavy);
+  } else {
+    b -= AHF_XCDS * per_f;
+    const int64_t w = (b % AHF_XCDS) * per_m + b / AHF_XCDS;
+    if (w >= T * T * nch) return; /* the whole workgroup */
+    gather_march<CAP, FULL>(v, w % T, (w / T) % T, T, w / (T * T), zn, S, pmask, p0, qp, descending, m2pd, kmax, dens,
+                            heavy, n_heavy);
+  }
+}
+
 /* inclusive prefix sum over the 64 lanes of a wavefront by DPP row shifts
  * (within each row of 16) and row broadcasts of lanes 15 and 31 into the
  * rows above (the GFX9 scan; register-only) */
@@ -1280,12 +1320,11 @@ __device__ inline int64_t readlane_i64(int64_t x, int l)
  * the lanes; exact ties take the parity of the running value, lane by lane.
  * The first lane whose step leaves the binade (or whose start is zero or
  * subnormal) takes the plain FP32 step, and the fold resumes after it.
- * Every round settles at least one lane.
+ * Every round settles at least one lane.  Lanes before `start` are settled.
  */
-__device__ float fold_wave(float d, double cv, int mm)
+__device__ float fold_wave(float d, double cv, int start, int mm)
 {
   const int lane = threadIdx.x & 63;
-  int start = 0;
   while (start < mm) {
     int ok;
     const int e = ahf_fold_exponent(d, &ok);
@@ -1330,196 +1369,334 @@ __device__ float fold_wave(float d, double cv, int mm)
 }
 
 /*
- * The contributing sources of heavy target n, flattened: lane j < 27 holds
- * source j of AHF's visiting order (ahf_axis_order on each axis, z outer),
- * its first entry q0, its entry count (0 when absent or masked out) and the
- * exclusive prefix of the counts; the return value is the total.
+ * Heavy targets (more than kmax contributions), in two lists of one array:
+ * those of at most AHF_HUGE contributions from its front, one wavefront
+ * each, the larger ones from its back, one workgroup each.
+ *
+ * A target's contributions are flattened across its 27 sources in AHF's
+ * visiting order (ahf_axis_order on each axis, z outer) and each source's
+ * list order.  A wavefront takes AHF_HV * 64 of them at a time, contribution
+ * base + 64*i + lane in register i.  As long as none is negative, none is an
+ * exact tie and the value stays inside its binade, the block moves the
+ * value's integer K by the sum of their steps (ahf_fold_step) in any order:
+ * no scan over the lanes and no chain.  A block that fails the test is folded
+ * 64 at a time in order (fold_wave): the first blocks, where the value runs
+ * from -1 through zero, and then about one per doubling of the density.
+ *
+ * Bound by the latency of the folds and of the loads, so by the wavefronts in
+ * flight: registers are held to 64 (8 wavefronts a SIMD; 81 registers and 5
+ * wavefronts take 5.2 ms where this takes 4.2).  Measured over the levels of a
+ * 192^3 clustered box (16,558 domain nodes above 384 contributions, the largest
+ * 570,521): 24 ms with one wavefront and fold_wave for every 64 contributions
+ * of a node, 4.2 ms now.
  */
-struct HeavySrc {
-  int64_t q0, cnt, off;
-  int ex, ey, ez;
+#define AHF_HV 4
+#define AHF_HBLK (64 * AHF_HV)
+#define AHF_HEAVY_BS 512
+#define AHF_HEAVY_NW (AHF_HEAVY_BS / 64)
+/* a target's sources in LDS: exclusive prefix of the entry counts (off[27]
+ * the total; an empty source shares its prefix with the next), the first
+ * entry, the offset code of each, and the centres of the nodes at -1, 0, +1
+ * along each axis */
+struct HeavyTab {
+  int64_t off[28], q0[27];
+  double c[3][3]; /* x, y, z */
+  int32_t code[27], pad;
 };
 
-__device__ inline int64_t heavy_sources(const level_view &v, const uint32_t *__restrict__ pmask,
-                                        const int64_t *__restrict__ p0, int64_t n, HeavySrc *hs)
+/* by one wavefront; returns the total */
+__device__ inline int64_t heavy_table(const level_view &v, const uint32_t *__restrict__ pmask,
+                                      const int64_t *__restrict__ p0, int64_t n, int descending, HeavyTab *T)
 {
   const int lane = threadIdx.x & 63;
   const int64_t o = n >> 3;
   const int c = (int)(n & 7);
-  hs->q0 = 0;
-  hs->cnt = 0;
-  hs->ex = hs->ey = hs->ez = 0;
+  int64_t X, Y, Z;
+  ahf_node_xyz(&v, o, c, &X, &Y, &Z);
+  int64_t q0 = 0, cnt = 0;
+  int code = 0;
   if (lane < 27) {
-    int64_t X, Y, Z;
-    ahf_node_xyz(&v, o, c, &X, &Y, &Z);
     int oz[3], oy[3], ox[3];
     ahf_axis_order(Z, v.L, oz);
     ahf_axis_order(Y, v.L, oy);
     ahf_axis_order(X, v.L, ox);
-    hs->ez = oz[lane / 9];
-    hs->ey = oy[(lane / 3) % 3];
-    hs->ex = ox[lane % 3];
-    const int64_t s = ahf_nbr_node(v.nbr, o, c, hs->ex, hs->ey, hs->ez);
-    if (s >= 0 && ((pmask[s] >> ((1 - hs->ez) * 9 + (1 - hs->ey) * 3 + (1 - hs->ex))) & 1u)) {
-      hs->q0 = p0[s];
-      hs->cnt = p0[s + 1] - hs->q0;
+    const int ez = oz[lane / 9], ey = oy[(lane / 3) % 3], ex = ox[lane % 3];
+    code = (ez + 1) * 16 + (ey + 1) * 4 + (ex + 1);
+    const int64_t s = ahf_nbr_node(v.nbr, o, c, ex, ey, ez);
+    if (s >= 0 && ((pmask[s] >> ((1 - ez) * 9 + (1 - ey) * 3 + (1 - ex))) & 1u)) {
+      q0 = p0[s];
+      cnt = p0[s + 1] - q0;
     }
   }
-  int64_t inc = hs->cnt;
+  int64_t inc = cnt;
 #pragma unroll
   for (int d = 1; d < 32; d <<= 1) {
     const int64_t t = __shfl_up(inc, d, 64);
     if (lane >= d) inc += t;
   }
-  hs->off = inc - hs->cnt;
-  return readlane_i64(inc, 26);
+  const int64_t total = readlane_i64(inc, 26);
+  if (lane < 27) {
+    T->off[lane] = inc - cnt;
+    T->q0[lane] = descending ? q0 + cnt - 1 : q0; /* the first in list order */
+    T->code[lane] = code;
+  } else if (lane == 27) {
+    T->off[27] = total;
+  } else if (lane >= 32 && lane < 41) {
+    const int a = (lane - 32) / 3, k = (lane - 32) % 3;
+    const int64_t W = a == 0 ? X : (a == 1 ? Y : Z);
+    T->c[a][k] = ahf_centre(ahf_wrap(W - 1 + k, v.L), (double)v.L);
+  }
+  __builtin_amdgcn_wave_barrier();
+  __threadfence_block();
+  return total;
+}
+
+/* the contributions [base, base + AHF_HBLK) of a target, 0.0 past its last
+ * (adding 0.0 leaves the value and K alone); j0: a source at or before the
+ * one holding `base`, the same on every lane, moved up to it */
+template <class Contrib>
+__device__ __forceinline__ void heavy_fetch(const HeavyTab *T, int64_t total, int64_t base, int descending, int &j0,
+                                            Contrib contrib, double cv[AHF_HV])
+{
+  const int lane = threadIdx.x & 63;
+  while (j0 < 26 && T->off[j0 + 1] <= base) j0++;
+  const bool one = T->off[j0 + 1] >= base + AHF_HBLK;
+#pragma unroll
+  for (int i = 0; i < AHF_HV; i++) {
+    const int64_t k = base + 64 * i + lane;
+    int j = j0;
+    if (!one) {
+      /* the last source whose prefix is at most k */
+#pragma unroll
+      for (int s = 16; s > 0; s >>= 1)
+        if (j + s < 27 && T->off[j + s] <= k) j += s;
+    }
+    cv[i] = 0.0;
+    if (k < total) {
+      const int64_t kk = k - T->off[j];
+      cv[i] = contrib(descending ? T->q0[j] - kk : T->q0[j] + kk, T->code[j]);
+    }
+  }
+}
+
+/* sum of the block's steps in the binade of exponent e over the wavefront;
+ * 0 when some contribution rules the block sum out */
+__device__ __forceinline__ int heavy_block_sum(const double cv[AHF_HV], int e, int64_t *S)
+{
+  const double scale = __longlong_as_double((long long)(1023 + 23 - e) << 52); /* 2^(23-e), -126 <= e <= 127 */
+  int32_t s = 0;
+  int ok = 1;
+#pragma unroll
+  for (int i = 0; i < AHF_HV; i++) {
+    int32_t r;
+    ok &= ahf_fold_step(cv[i], scale, &r) & (int)(cv[i] >= 0.0);
+    s += r; /* at most 2^22 each */
+  }
+  /* at most 2^31 over the wavefront: exact modulo 2^32 */
+  *S = (int64_t)(uint32_t)__builtin_amdgcn_readlane(wave_incl_scan_dpp(s), 63);
+  return __ballot(!ok) == 0ull;
+}
+
+/* K of a normal float in its binade, and back */
+__device__ __forceinline__ int64_t heavy_K(float d)
+{
+  const uint32_t u = __float_as_uint(d);
+  const int64_t m = (int64_t)((u & 0x7FFFFFu) | 0x800000u);
+  return (u >> 31) ? -m : m;
+}
+__device__ __forceinline__ float heavy_value(int64_t K, int e) { return ldexpf((float)(int32_t)K, e - 23); }
+
+/*
+ * 64 contributions in order (lanes [0, mm), the other lanes 0.0): rounds of a
+ * scan of the steps over the lanes, each up to the first lane that ends on or
+ * beyond the binade's edge, which takes the plain FP32 step; from a lane with
+ * an exact tie (or a NaN) on by fold_wave, which knows the ties' parities.
+ * A round is about 60 instructions; fold_wave's, on 64-bit integers, three
+ * times that.
+ */
+__device__ __forceinline__ float heavy_fold1(float d, double cv, int mm)
+{
+  const int lane = threadIdx.x & 63;
+  for (int start = 0; start < mm;) {
+    int normal;
+    const int e = ahf_fold_exponent(d, &normal);
+    int bad = start;
+    if (normal) {
+      const double scale = __longlong_as_double((long long)(1023 + 23 - e) << 52);
+      int32_t r;
+      const int ok = ahf_fold_step(cv, scale, &r);
+      const bool act = lane >= start;
+      const int32_t P = wave_incl_scan_dpp(act ? r : 0); /* at most 2^28 */
+      const int32_t K0 = (int32_t)heavy_K(d), K = K0 + P, A = K < 0 ? -K : K;
+      /* strictly inside, of d's own sign: the double sum lay inside as well */
+      const bool in = ok && A > (1 << 23) && A < (1 << 24) && (K ^ K0) >= 0;
+      const uint64_t out = __ballot(act && lane < mm && !in);
+      bad = out ? __builtin_ctzll(out) : mm;
+      if (bad > start) d = heavy_value(K0 + (int64_t)__builtin_amdgcn_readlane(P, bad - 1), e);
+      if (bad == mm) break;
+      /* |c| of 2^22 ulps or more leaves the step to plain FP32 as well */
+      const double c = readlane_d(cv, bad);
+      if (!__builtin_amdgcn_readlane(ok, bad) && !(fabs(c * scale) >= 4194304.0)) return fold_wave(d, cv, bad, mm);
+    }
+    d = (float)((double)d + readlane_d(cv, bad));
+    start = bad + 1;
+  }
+  return d;
+}
+
+/* the same one contribution after the other, the lanes read in turn: about 40
+ * cycles each.  A target's first 64 run from -1 through zero and cross a
+ * binade every few contributions; a round of heavy_fold1 for each crossing,
+ * about 600 cycles, costs them four times as much. */
+__device__ __forceinline__ float heavy_serial(float d, double cv, int mm)
+{
+  int l = 0;
+  for (; l + 8 <= mm; l += 8)
+#pragma unroll
+    for (int i = 0; i < 8; i++) d = (float)((double)d + readlane_d(cv, l + i));
+  for (; l < mm; l++) d = (float)((double)d + readlane_d(cv, l));
+  return d;
+}
+
+/* the block folded 64 at a time, in order (cv is used up: rotated through
+ * its first register, so the fold is there once and not AHF_HV times);
+ * first: the target's first block */
+__device__ __forceinline__ float heavy_fold64(float d, double cv[AHF_HV], int64_t left, bool first)
+{
+#pragma unroll 1
+  for (int done = 0; done < AHF_HBLK && done < left; done += 64) {
+    const int mm = (int)(left - done < 64 ? left - done : 64);
+    d = first && done == 0 ? heavy_serial(d, cv[0], mm) : heavy_fold1(d, cv[0], mm);
+#pragma unroll
+    for (int i = 0; i + 1 < AHF_HV; i++) cv[i] = cv[i + 1];
+  }
+  return d;
+}
+
+template <class Contrib>
+__device__ float heavy_wave(const HeavyTab *T, int64_t total, int descending, Contrib contrib)
+{
+  float d = -1.0f;
+  int j0 = 0;
+  for (int64_t base = 0; base < total; base += AHF_HBLK) {
+    double cv[AHF_HV];
+    heavy_fetch(T, total, base, descending, j0, contrib, cv);
+    int ok;
+    const int e = ahf_fold_exponent(d, &ok);
+    if (ok) {
+      int64_t S;
+      ok = heavy_block_sum(cv, e, &S);
+      const int64_t K = heavy_K(d);
+      ok = ok && ahf_fold_block_in(K, S);
+      if (ok) d = heavy_value(K + S, e);
+    }
+    if (!ok) d = heavy_fold64(d, cv, total - base, base == 0);
+  }
+  return d;
+}
+
+/* the same by the whole workgroup, its wavefronts taking consecutive blocks:
+ * every wavefront sums its block in the binade the value has now, all of them
+ * add the sums up in order to the first block that fails, that one is folded
+ * by its wavefront, and the blocks after it are summed again in the binade
+ * the value has then (at most AHF_HEAVY_NW rounds).  d and every branch
+ * around a barrier are the same on all threads.  The rounds alternate
+ * between two sets of words: a wavefront writes one of them only after the
+ * barrier that follows every reading of the round before. */
+struct HeavyRound {
+  uint32_t S[2][AHF_HEAVY_NW];
+  int32_t ok[2][AHF_HEAVY_NW];
+  float d[2];
+};
+
+template <class Contrib>
+__device__ float heavy_group(const HeavyTab *T, int64_t total, int descending, HeavyRound *R, int &turn,
+                             Contrib contrib)
+{
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  float d = -1.0f;
+  int j0 = 0;
+  for (int64_t base = 0; base < total; base += (int64_t)AHF_HEAVY_NW * AHF_HBLK) {
+    double cv[AHF_HV];
+    const int64_t wbase = base + (int64_t)w * AHF_HBLK;
+    heavy_fetch(T, total, wbase, descending, j0, contrib, cv);
+    for (int w0 = 0; w0 < AHF_HEAVY_NW; turn ^= 1) {
+      int normal;
+      const int e = ahf_fold_exponent(d, &normal);
+      int64_t S = 0;
+      int ok = 0;
+      if (normal && w >= w0) ok = heavy_block_sum(cv, e, &S);
+      if (lane == 0) {
+        R->S[turn][w] = (uint32_t)S;
+        R->ok[turn][w] = ok;
+      }
+      __syncthreads();
+      int wb = w0;
+      if (normal) {
+        /* the value after each block from w0 on, one per lane (a sum of 2^24
+         * or more, capped there, fails as it is); the first that fails */
+        const bool mine = lane >= w0 && lane < AHF_HEAVY_NW;
+        const uint32_t Sl = mine ? R->S[turn][lane] : 0u;
+        const int okl = mine ? R->ok[turn][lane] : 0;
+        const int32_t P = wave_incl_scan_dpp((int32_t)(Sl < (1u << 24) ? Sl : (1u << 24)));
+        const int64_t K = heavy_K(d);
+        const uint64_t fail = __ballot(mine && !(okl && ahf_fold_block_in(K, (int64_t)P)));
+        wb = fail ? __builtin_ctzll(fail) : AHF_HEAVY_NW;
+        if (wb > w0) d = heavy_value(K + (int64_t)__builtin_amdgcn_readlane(P, wb - 1), e);
+      }
+      if (wb < AHF_HEAVY_NW) {
+        if (w == wb) {
+          const float f = heavy_fold64(d, cv, total - wbase, wbase == 0);
+          if (lane == 0) R->d[turn] = f;
+        }
+        __syncthreads();
+        d = R->d[turn];
+      }
+      w0 = wb + 1;
+    }
+  }
+  return d;
 }
 
 /*
- * The source (lane of heavy_sources) and entry of flat contribution k =
- * base + lane, for one round of 64.  j0, uniform, is the source holding
- * contribution base and is advanced round by round; the few sources that
- * start inside the round are taken from their lanes with readlane (scalar
- * reads, no cross-lane shuffles).  A source holds k when it is the last
- * whose prefix is at most k (empty sources share their prefix with the next).
+ * Exact-order density of the heavy targets: first the huge ones by
+ * workgroups, then the others by wavefronts.  Every level's heavy targets
+ * read the 16-byte position records, consecutive lanes consecutive records,
+ * and form the weights again (about 40 FP64 instructions): over 80-byte
+ * weight records a wavefront's loads touch five times the cache lines.
  */
-struct HeavyLane {
-  int64_t q;
-  int ex, ey, ez;
-  bool in;
-};
-
-__device__ inline HeavyLane heavy_lane(const HeavySrc &hs, int64_t total, int64_t base, int &j0, int descending)
+__global__ void __launch_bounds__(AHF_HEAVY_BS, 8) k_gather_heavy(level_view v, const uint32_t *__restrict__ pmask,
+                                                               const int64_t *__restrict__ p0,
+                                                               const ahf_q4 *__restrict__ qp, int descending,
+                                                               double m2pd, float *__restrict__ dens,
+                                                               const uint32_t *__restrict__ heavy,
+                                                               const uint32_t *__restrict__ n_heavy)
 {
-  const int lane = threadIdx.x & 63;
-  const int64_t k = base + lane;
-  while (j0 < 26 && readlane_i64(hs.off, j0 + 1) <= base) j0++;
-  const int64_t kend = (base + 63 < total - 1) ? base + 63 : total - 1;
-  const int code = hs.ex + 1 + 3 * (hs.ey + 1) + 9 * (hs.ez + 1);
-  int64_t q0 = readlane_i64(hs.q0, j0), cnt = readlane_i64(hs.cnt, j0), off = readlane_i64(hs.off, j0);
-  int cd = __builtin_amdgcn_readlane(code, j0);
-  for (int j = j0 + 1; j < 27; j++) {
-    const int64_t oj = readlane_i64(hs.off, j);
-    if (oj > kend) break;
-    const int64_t qj = readlane_i64(hs.q0, j), cj = readlane_i64(hs.cnt, j);
-    const int dj = __builtin_amdgcn_readlane(code, j);
-    const bool mine = k >= oj;
-    q0 = mine ? qj : q0;
-    cnt = mine ? cj : cnt;
-    off = mine ? oj : off;
-    cd = mine ? dj : cd;
-  }
-  HeavyLane r;
-  const int64_t kk = k - off;
-  r.in = k < total;
-  r.q = descending ? q0 + cnt - 1 - kk : q0 + kk;
-  r.ex = cd % 3 - 1;
-  r.ey = (cd / 3) % 3 - 1;
-  r.ez = cd / 9 - 1;
-  return r;
-}
-
-/* exact-order density of the heavy targets, one wavefront per target: the
- * node's contributions, source by source in AHF's order and each source's
- * entries in list order, are taken 64 at a time (one per lane) and folded
- * into the FP32 node value (fold_wave) */
-__global__ void __launch_bounds__(AHF_BLOCK) k_gather_heavy(level_view v, const uint32_t *__restrict__ pmask,
-                                                            const int64_t *__restrict__ p0,
-                                                            const ahf_w9 *__restrict__ W, int descending,
-                                                            float *__restrict__ dens,
-                                                            const uint32_t *__restrict__ heavy,
-                                                            const uint32_t *__restrict__ n_heavy)
-{
-  const int lane = threadIdx.x & 63;
-  const int64_t gw = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int64_t nh = (int64_t)*n_heavy;
-  for (int64_t i = gw; i < nh; i += nw) {
-    const int64_t n = heavy[i];
-    HeavySrc hs;
-    const int64_t total = heavy_sources(v, pmask, p0, n, &hs);
-    float d = -1.0f;
-    /* the next round's weights are loaded before this round is folded */
-    int j0 = 0;
-    auto fetch = [&](int64_t base, double &b0, double &b1, double &b2) {
-      const HeavyLane hl = heavy_lane(hs, total, base, j0, descending);
-      b0 = b1 = b2 = 0.0;
-      if (hl.in) {
-        const double *w = reinterpret_cast<const double *>(W + hl.q);
-        b0 = w[1 - hl.ez];
-        b1 = w[3 + (1 - hl.ey)];
-        b2 = w[6 + (1 - hl.ex)];
-      }
-    };
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    if (total > 0) fetch(0, a0, a1, a2);
-    for (int64_t base = 0; base < total; base += 64) {
-      /* lanes past the end fold nothing (mm below) */
-      const double cv = (a0 * a1) * a2;
-      double b0 = 0.0, b1 = 0.0, b2 = 0.0;
-      if (base + 64 < total) fetch(base + 64, b0, b1, b2);
-      d = fold_wave(d, cv, (int)(total - base < 64 ? total - base : 64));
-      a0 = b0;
-      a1 = b1;
-      a2 = b2;
-    }
-    if (lane == 0) dens[n] = d;
-  }
-}
-
-/* k_gather_heavy over position records (dense levels) */
-__global__ void __launch_bounds__(AHF_BLOCK) k_gather_heavy_q(level_view v, const uint32_t *__restrict__ pmask,
-                                                            const int64_t *__restrict__ p0,
-                                                            const ahf_q4 *__restrict__ qp, int descending,
-                                                            double m2pd, float *__restrict__ dens,
-                                                            const uint32_t *__restrict__ heavy,
-                                                            const uint32_t *__restrict__ n_heavy)
-{
-  const int lane = threadIdx.x & 63;
-  const int64_t gw = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int64_t nh = (int64_t)*n_heavy;
+  __shared__ HeavyTab s_tab[AHF_HEAVY_NW];
+  __shared__ HeavyRound s_round;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  HeavyTab *T = s_tab + w;
+  const int64_t n_huge = (int64_t)n_heavy[1], n_rest = (int64_t)n_heavy[0], nn = 8 * v.n_oct;
   const double L = (double)v.L;
-  for (int64_t i = gw; i < nh; i += nw) {
+  auto contrib = [=](int64_t q, int code) {
+    const ahf_q4 r = qp[q];
+    const int ez = (code >> 4) - 1, ey = ((code >> 2) & 3) - 1, ex = (code & 3) - 1;
+    const double wz = TscRt(-ez)(ahf_pn_sep(r.z, T->c[2][ez + 1], L));
+    const double wy = TscRt(-ey)(ahf_pn_sep(r.y, T->c[1][ey + 1], L));
+    const double wx = TscRt(-ex)(ahf_pn_sep(r.x, T->c[0][ex + 1], L));
+    return ((m2pd * wz) * wy) * wx;
+  };
+  int turn = 0;
+  for (int64_t i = blockIdx.x; i < n_huge; i += gridDim.x) {
+    const int64_t n = heavy[nn - 1 - i];
+    const int64_t total = heavy_table(v, pmask, p0, n, descending, T);
+    const float d = heavy_group(T, total, descending, &s_round, turn, contrib);
+    if (threadIdx.x == 0) dens[n] = d;
+  }
+  for (int64_t i = (int64_t)w * gridDim.x + blockIdx.x; i < n_rest; i += (int64_t)gridDim.x * AHF_HEAVY_NW) {
     const int64_t n = heavy[i];
-    int64_t X, Y, Z;
-    ahf_node_xyz(&v, n >> 3, (int)(n & 7), &X, &Y, &Z);
-    double cxv[3], cyv[3], czv[3];
-    ahf_centres3(X, v.L, cxv);
-    ahf_centres3(Y, v.L, cyv);
-    ahf_centres3(Z, v.L, czv);
-    HeavySrc hs;
-    const int64_t total = heavy_sources(v, pmask, p0, n, &hs);
-    float d = -1.0f;
-    /* the next round's records are loaded before this round is folded */
-    int ex = 0, ey = 0, ez = 0;
-    bool in = false;
-    ahf_q4 e4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    int j0 = 0;
-    auto fetch = [&](int64_t base, ahf_q4 &rec, int &fx, int &fy, int &fz, bool &ok) {
-      const HeavyLane hl = heavy_lane(hs, total, base, j0, descending);
-      fx = hl.ex;
-      fy = hl.ey;
-      fz = hl.ez;
-      ok = hl.in;
-      if (ok) rec = qp[hl.q];
-    };
-    if (total > 0) fetch(0, e4, ex, ey, ez, in);
-    for (int64_t base = 0; base < total; base += 64) {
-      const double cv = in ? ahf_contrib(m2pd, ahf_pn_sep(e4.x, cxv[ex + 1], L), ahf_pn_sep(e4.y, cyv[ey + 1], L),
-                                         ahf_pn_sep(e4.z, czv[ez + 1], L), -ex, -ey, -ez)
-                           : 0.0;
-      ahf_q4 n4 = {0.0f, 0.0f, 0.0f, 0.0f};
-      int nx = 0, ny = 0, nz = 0;
-      bool nin = false;
-      if (base + 64 < total) fetch(base + 64, n4, nx, ny, nz, nin);
-      d = fold_wave(d, cv, (int)(total - base < 64 ? total - base : 64));
-      e4 = n4;
-      ex = nx;
-      ey = ny;
-      ez = nz;
-      in = nin;
-    }
+    const int64_t total = heavy_table(v, pmask, p0, n, descending, T);
+    const float d = heavy_wave(T, total, descending, contrib);
     if (lane == 0) dens[n] = d;
   }
 }
@@ -1923,12 +2100,44 @@ static level_view make_view(const DevLevel &l)
 
 /* bucket entries per node from which a level counts as dense */
 #define AHF_DENSE_ENTRIES_PER_NODE 3
-/* heavy-node workgroups: 7 wavefronts per SIMD on 256 CUs, each wavefront
- * folding one node at a time */
-#define AHF_HEAVY_BLOCKS 1792
-/* nodes with more contributions than this go to the heavy kernels */
-#define AHF_KMAX_BIG 384u   /* levels of 2^21 nodes or more */
-#define AHF_KMAX_SMALL 96u
+/* heavy-node workgroups: four of 8 wavefronts on each of 256 CUs, all resident */
+#define AHF_HEAVY_BLOCKS 1024
+/* nodes with more contributions than this go to the heavy kernel: on levels
+ * that do not march, and at most on any */
+#define AHF_KMAX_SMALL 96
+#define AHF_KMAX_TOP 2000
+
+/* a level that holds every octet takes the staged plane walk, unless it is
+ * so small that its few workgroups, each marching through planes, take longer
+ * than a lane or a wavefront per node */
+/* L = 32 at 8 and at 1 entries a node: 0.54 ms marched, 0.09 ms not; L = 50:
+ * 0.58 ms marched (deposit of all its levels), 0.96 ms not */
+#define AHF_MARCH_MIN_L 40
+static bool marches(const ahfgpu_ctx *c, int64_t L, int64_t n_oct)
+{
+  return c->gather_mode == AHFGPU_GATHER_AUTO && L >= AHF_MARCH_MIN_L && n_oct == (L / 2) * (L / 2) * (L / 2);
+}
+
+/* target planes per marching workgroup: a workgroup walks zn + 2 source
+ * planes, and about AHF_MARCH_FILL of them are resident at once, so on small
+ * levels the fewest rounds of planes (L = 64: 496 workgroups of 2 planes take
+ * 0.15 ms, 128 of 8 planes 0.37).  Larger levels have workgroups to spare and
+ * take the planes that re-read least. */
+#define AHF_MARCH_FILL 512
+static int64_t march_planes(int64_t L, int64_t side)
+{
+  if (L >= 128) return L <= 128 ? 8 : 16;
+  int64_t best = 0, cost = 0;
+  for (int64_t zn = 1; zn <= 16; zn *= 2) {
+    const int64_t wg = side * side * ((L - 2 + zn - 1) / zn);
+    const int64_t c = (wg + AHF_MARCH_FILL - 1) / AHF_MARCH_FILL * (zn + 2);
+    if (!best || c < cost) {
+      best = zn;
+      cost = c;
+    }
+  }
+  return best;
+}
 
 /*
  * Exact-order gather of one level over its n_ent bucket entries: the octets
@@ -1938,7 +2147,7 @@ static level_view make_view(const DevLevel &l)
  *  - sparse levels: a TSC weight record per entry and the flat walk
  *    (k_gather_light), which keeps a wavefront's lanes busy when buckets
  *    hold a particle or two;
- * and one wavefront per node with more than kmax contributions.  Every
+ * and by wavefronts the nodes with more than kmax contributions.  Every
  * choice gives the same bits.  Needs pmask.
  */
 static int gather_level(ahfgpu_ctx *c, DevLevel &l, int64_t n_ent, int descending, bool timed)
@@ -1947,27 +2156,22 @@ static int gather_level(ahfgpu_ctx *c, DevLevel &l, int64_t n_ent, int descendin
   level_view v = make_view(l);
   Arena &A = c->arena;
   /* a level that holds every octet takes the staged plane walk */
-  const bool slab = c->gather_mode == AHFGPU_GATHER_AUTO && l.L % AHF_SLAB == 0 &&
-                    no == (l.L / 2) * (l.L / 2) * (l.L / 2);
+  const bool slab = marches(c, l.L, no);
   const bool dense = slab || c->gather_mode == AHFGPU_GATHER_SOURCE ||
                      ((c->gather_mode == AHFGPU_GATHER_AUTO || c->gather_mode == AHFGPU_GATHER_WAVE) &&
                       n_ent >= AHF_DENSE_ENTRIES_PER_NODE * nn);
   l.dens = A.get<float>(nn);
-  l.qp = nullptr;
-  l.W = nullptr;
-  if (dense)
-    l.qp = A.get<ahf_q4>(n_ent > 0 ? n_ent : 1);
-  else
-    l.W = A.get<ahf_w9>(n_ent > 0 ? n_ent : 1);
+  l.qp = A.get<ahf_q4>(n_ent > 0 ? n_ent : 1);
+  l.W = dense ? nullptr : A.get<ahf_w9>(n_ent > 0 ? n_ent : 1);
   uint32_t *heavy = A.get<uint32_t>(nn);
-  if (!l.dens || !(dense ? (void *)l.qp : (void *)l.W) || !heavy) return AHFGPU_ENOMEM;
-  uint32_t *n_heavy = (uint32_t *)(c->d_anomaly + 1);
-  hipMemsetAsync(n_heavy, 0, sizeof(uint32_t), c->st);
+  if (!l.dens || !l.qp || (!dense && !l.W) || !heavy) return AHFGPU_ENOMEM;
+  uint32_t *n_heavy = (uint32_t *)(c->d_anomaly + 4); /* two counts */
+  hipMemsetAsync(n_heavy, 0, 2 * sizeof(uint32_t), c->st);
   hipEvent_t e0 = timed ? c->timer_begin() : nullptr;
   if (dense)
     LAUNCH(k_prep_q, n_ent, l.node_p0 + nn, n_ent, l.plist, c->px, c->py, c->pz, l.qp);
   else
-    LAUNCH(k_prep, n_ent, v, l.node_p0 + nn, n_ent, l.pnode, l.plist, c->px, c->py, c->pz, l.m2pd, l.W);
+    LAUNCH(k_prep, n_ent, v, l.node_p0 + nn, n_ent, l.pnode, l.plist, c->px, c->py, c->pz, l.m2pd, l.W, l.qp);
   if (!l.tord) {
     /* no order inherited from a coarser level: sort the octets' Morton keys */
     uint64_t *mk0 = A.get<uint64_t>(no), *mk1 = A.get<uint64_t>(no);
@@ -1986,30 +2190,30 @@ static int gather_level(ahfgpu_ctx *c, DevLevel &l, int64_t n_ent, int descendin
   hipEvent_t e1 = timed ? c->timer_begin() : nullptr;
   const int64_t per_xcd = (nblk(nn) + AHF_XCDS - 1) / AHF_XCDS;
   const dim3 grid((unsigned)(AHF_XCDS * per_xcd));
-  /* long lanes in a small launch leave the chip idle: hand them to the
-   * wavefront-per-node kernel sooner */
-  const uint32_t kmax_big = c->kmax_big > 0 ? (uint32_t)c->kmax_big : AHF_KMAX_BIG;
-  const uint32_t kmax_small = c->kmax_small > 0 ? (uint32_t)c->kmax_small : AHF_KMAX_SMALL;
-  const uint32_t kmax = c->gather_mode == AHFGPU_GATHER_WAVE ? 0u : nn >= ((int64_t)1 << 21) ? kmax_big : kmax_small;
-  static_assert(AHF_KMAX_BIG < 4096 && AHF_KMAX_SMALL < 4096, "the march's queue words hold counts below 4096");
+  /* a lane's chain holds its whole wavefront, so a node goes to the heavy
+   * kernel once it has well more contributions than its neighbours: half as
+   * much again as the marching level's mean of 27 per entry of a node, and
+   * AHF_KMAX_SMALL on the others (the schedule's kmax_big and kmax_small set the
+   * threshold itself, for levels of 2^21 nodes or more and for smaller ones) */
+  const int64_t mean = 27 * n_ent / (nn > 0 ? nn : 1);
+  const uint32_t kdef =
+      slab ? (uint32_t)std::min<int64_t>(AHF_KMAX_TOP, std::max<int64_t>(AHF_KMAX_SMALL, mean + mean / 2)) : AHF_KMAX_SMALL;
+  const int32_t kset = nn >= ((int64_t)1 << 21) ? c->kmax_big : c->kmax_small;
+  const uint32_t kmax = c->gather_mode == AHFGPU_GATHER_WAVE ? 0u : kset > 0 ? (uint32_t)kset : kdef;
+  static_assert(AHF_KMAX_TOP < 4096, "the march's queue words hold counts below 4096");
   if (slab) {
     /* the planes 1..L-2 march, the two face planes take the per-plane walk */
-    const int64_t side = l.L / AHF_SLAB;
-    const int64_t zn = c->march_zn > 0 ? c->march_zn : l.L <= 128 ? 8 : 16, nch = (l.L - 2 + zn - 1) / zn;
+    const int64_t side = (l.L + AHF_SLAB - 1) / AHF_SLAB;
+    const int64_t zn = c->march_zn > 0 ? c->march_zn : march_planes(l.L, side), nch = (l.L - 2 + zn - 1) / zn;
     const int64_t per_m = (side * side * nch + AHF_XCDS - 1) / AHF_XCDS;
     const int64_t per_f = (side * side * 2 + AHF_XCDS - 1) / AHF_XCDS;
-    const dim3 mgrid((unsigned)(AHF_XCDS * per_m)), fgrid((unsigned)(AHF_XCDS * per_f));
-    if (n_ent >= 2 * nn) {
-      hipLaunchKernelGGL((k_gather_march<AHF_SLAB_CAP_BIG, false>), mgrid, dim3(AHF_BLOCK), 0, c->st, v, per_m, zn,
+    const dim3 fgrid((unsigned)(AHF_XCDS * (per_f + per_m)));
+    if (n_ent >= 2 * nn)
+      hipLaunchKernelGGL((k_gather_full<AHF_FULL_CAP_BIG, false>), fgrid, dim3(AHF_BLOCK), 0, c->st, v, per_f, per_m, zn,
                          l.pmask, l.node_p0, l.qp, descending, l.m2pd, kmax, l.dens, heavy, n_heavy);
-      hipLaunchKernelGGL((k_gather_slab<AHF_SLAB_CAP_BIG, false>), fgrid, dim3(AHF_BLOCK), 0, c->st, v, per_f, l.pmask,
-                         l.node_p0, l.qp, descending, l.m2pd, kmax, l.dens, heavy, n_heavy, 1);
-    } else {
-      hipLaunchKernelGGL((k_gather_march<AHF_MARCH_CAP_SMALL, true>), mgrid, dim3(AHF_BLOCK), 0, c->st, v, per_m, zn,
-                         l.pmask, l.node_p0, l.qp, descending, l.m2pd, kmax, l.dens, heavy, n_heavy);
-      hipLaunchKernelGGL((k_gather_slab<AHF_SLAB_CAP_SMALL, true>), fgrid, dim3(AHF_BLOCK), 0, c->st, v, per_f, l.pmask,
-                         l.node_p0, l.qp, descending, l.m2pd, kmax, l.dens, heavy, n_heavy, 1);
-    }
+    else
+      hipLaunchKernelGGL((k_gather_full<AHF_FULL_CAP_SMALL, true>), fgrid, dim3(AHF_BLOCK), 0, c->st, v, per_f, per_m,
+                         zn, l.pmask, l.node_p0, l.qp, descending, l.m2pd, kmax, l.dens, heavy, n_heavy);
   } else if (dense)
     hipLaunchKernelGGL(k_gather_src, grid, dim3(AHF_BLOCK), 0, c->st, v, tord, per_xcd, l.pmask, l.node_p0, l.qp,
                        descending, l.m2pd, kmax, l.dens, heavy, n_heavy);
@@ -2022,12 +2226,8 @@ static int gather_level(ahfgpu_ctx *c, DevLevel &l, int64_t n_ent, int descendin
                        l.W, descending, kmax, l.dens, heavy, n_heavy);
   if (timed) c->timer_end(e1, TIMER_GATHER, 12.0 * (double)n_ent + 13.0 * (double)nn);
   hipEvent_t e2 = timed ? c->timer_begin() : nullptr;
-  if (dense)
-    hipLaunchKernelGGL(k_gather_heavy_q, dim3(AHF_HEAVY_BLOCKS), dim3(AHF_BLOCK), 0, c->st, v, l.pmask, l.node_p0, l.qp,
-                       descending, l.m2pd, l.dens, heavy, n_heavy);
-  else
-    hipLaunchKernelGGL(k_gather_heavy, dim3(AHF_HEAVY_BLOCKS), dim3(AHF_BLOCK), 0, c->st, v, l.pmask, l.node_p0, l.W,
-                       descending, l.dens, heavy, n_heavy);
+  hipLaunchKernelGGL(k_gather_heavy, dim3(AHF_HEAVY_BLOCKS), dim3(AHF_HEAVY_BS), 0, c->st, v, l.pmask, l.node_p0, l.qp,
+                     descending, l.m2pd, l.dens, heavy, n_heavy);
   if (timed) c->timer_end(e2, TIMER_HEAVY, 0.0);
   return 0;
 }
@@ -2212,7 +2412,7 @@ static int refine_level(ahfgpu_ctx *c, int ci)
    * sizes the deposit's records and launches, and the count is read with
    * the next level's sizes */
   const int gm = c->gather_mode;
-  const bool full_f = gm == AHFGPU_GATHER_AUTO && f.L % AHF_SLAB == 0 && f.n_oct == (f.L / 2) * (f.L / 2) * (f.L / 2);
+  const bool full_f = marches(c, f.L, f.n_oct);
   const bool decided = gm == AHFGPU_GATHER_FLAT || gm == AHFGPU_GATHER_FLAT_WIDE || gm == AHFGPU_GATHER_SOURCE || full_f ||
                        nent < AHF_DENSE_ENTRIES_PER_NODE * nn2;
   int64_t nent_f = nent;

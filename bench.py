@@ -483,8 +483,8 @@ def main():
         "stage_ms": stage_ms,
         "dominant_stage": dom,
         "roofline": {
-            "kernel": ("exact-order TSC deposit, one timed launch per grid level: k_gather_march + "
-                       "k_gather_slab (face planes) on levels holding every octet, k_gather_light on the others"),
+            "kernel": ("exact-order TSC deposit, one timed launch per grid level: k_gather_full "
+                       "on levels holding every octet, k_gather_light on the others"),
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,

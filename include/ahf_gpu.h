@@ -316,8 +316,9 @@ typedef struct {
   int64_t prof_split;  /* HaloProfiles: haloes of this many members or more on four wavefronts (-1: none); 2048 */
   int64_t big_halo;    /* unbinding: haloes of this many members or more on 512-thread workgroups; 2048 */
   int64_t wave_halo;   /* unbinding: haloes below this many members on one wavefront; 512 */
-  int32_t kmax_big;    /* deposit: nodes with more contributions folded by a wavefront (levels of 2^21 nodes or more); 384 */
-  int32_t kmax_small;  /* ... on smaller levels; 96 */
+  int32_t kmax_big;    /* deposit: nodes with more contributions folded by wavefronts (levels of 2^21 nodes or more);
+                          1.5 times the level's mean, at least 96 */
+  int32_t kmax_small;  /* ... on smaller levels; the same */
   int32_t march_zn;    /* deposit: target planes per march workgroup (8 or 16); by level size */
   int32_t graph_batch; /* split unbinding: iteration graph replays between done checks; 4 */
   int32_t split_spec;  /* split unbinding: passes settling all tiles at once before the sequential walk

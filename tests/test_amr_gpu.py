@@ -93,6 +93,43 @@ def test_staged_plane_overflow(oracle, ctx, tmp_path, n_bg, clump):
     _check(oracle, ctx, snap, tmp_path, f"clump{n_bg}_{clump}", 0)
 
 
+@pytest.mark.parametrize("L,per_node,clump", [(38, 3, 0), (40, 3, 4000), (42, 1, 900), (48, 3, 4000), (50, 1, 900),
+                                              (50, 4, 6000), (62, 1, 900), (64, 2, 4000)])
+def test_marched_levels(oracle, ctx, tmp_path, L, per_node, clump):
+    """domain grids on both sides of the size from which a level that holds
+    every octet marches, with whole and partial tiles, both staging forms,
+    and a clump beyond a plane's staged slots at the corner of the box (and
+    on the face planes) and one inside"""
+    rng = np.random.default_rng(L * 10 + per_node)
+    parts = [rng.random((per_node * L ** 3, 3))]
+    for c in ([0.0, 0.999, 0.0], [0.31, 0.5, 0.62]):
+        parts.append((np.array(c) + 1.5 / L * rng.standard_normal((clump, 3))) % 1.0)
+    pos = np.concatenate(parts).astype(np.float32)
+    pos[pos >= 1.0] = 0.0
+    snap = str(tmp_path / "m.snap")
+    dumps.write_snapshot(snap, pos, L_dom=L, L_max=L << 4, Nth_dom=1.5 * per_node, Nth_ref=4.0)
+    _check(oracle, ctx, snap, tmp_path, f"march{L}_{per_node}_{clump}", 0)
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("L,clump,dyadic", [(16, 2047, False), (16, 9000, False), (10, 20000, False), (16, 70000, False),
+                                            (16, 20000, True), (10, 4000, True)])
+def test_huge_nodes(oracle, ctx, tmp_path, L, clump, dyadic, mode):
+    """nodes on both sides of the contribution count from which a workgroup
+    folds a node, over position and weight records, blocks of every length;
+    positions on a dyadic lattice make steps that are exact halves"""
+    rng = np.random.default_rng(clump + L)
+    c = np.array([0.5 + 0.3 / L, 0.02, 0.31])
+    cl = c + rng.standard_normal((clump, 3)) * np.array([0.05, 0.2, 0.1])[rng.integers(0, 3, (clump, 1))] / L
+    if dyadic:
+        cl = np.round(cl * 1024.0) / 1024.0
+    pos = np.concatenate([rng.random((500, 3)), cl % 1.0]).astype(np.float32)
+    pos[pos >= 1.0] = 0.0
+    snap = str(tmp_path / "huge.snap")
+    dumps.write_snapshot(snap, pos, L_dom=L, L_max=L << 6, Nth_dom=4.0, Nth_ref=4.0)
+    _check(oracle, ctx, snap, tmp_path, f"huge{L}_{clump}_{dyadic}", mode)
+
+
 @pytest.mark.parametrize("sched", [dict(kmax_big=8, kmax_small=8, march_zn=8), dict(kmax_big=1000, kmax_small=300, march_zn=16)])
 @pytest.mark.parametrize("cfg,side,seed", [(1, 64, 1001), (3, 64, 1003)])
 def test_schedule_variants(oracle, snapgen, ctx, tmp_path, cfg, side, seed, sched):

@@ -65,6 +65,19 @@ def test_wavefront_fold_replay(tmp_path):
         assert '"mismatches": 0' in r.stdout
 
 
+def test_heavy_block_sum(tmp_path):
+    """the heavy kernels' block sum (steps of a binade added in any order)
+    against AHF's sequential FP32 accumulation: every block that its test
+    accepts is bit-identical, with ties, negative contributions and binade
+    edges among the blocks"""
+    exe = str(tmp_path / "block_sum_check")
+    subprocess.run(["gcc", "-std=c11", "-O2", "-ffp-contract=off", "-Wno-unused-function", "-o", exe,
+                    os.path.join(HERE, "emu", "block_sum_check.c"), "-lm"], check=True)
+    for seed in (1, 2):
+        r = subprocess.run([exe, "200000", str(seed)], capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:] + r.stdout
+
+
 def test_fold64_replay(tmp_path):
     """an FP64 running-sum fold (integer steps on a binade's grid,
     exact ties by parity, plain steps across binades and from zero or
