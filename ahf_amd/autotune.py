@@ -37,9 +37,9 @@ CANDIDATES = {
     "kmax_big": [0, 384, 192, 256, 512, 768, 1024],
     "kmax_small": [0, 96, 48, 64, 128, 192],
     "march_zn": [0, 8, 16],
-    "big_halo": [2048, 1024, 4096, 8192],
-    "wave_halo": [512, 256, 1024],
-    "split_min": [16384, 4096, 8192, 32768, 65536, -1],
+    "big_halo": [0, 512, 1024],
+    "wave_halo": [0, 128, 256],
+    "split_min": [0, 4097, 8192, 16384, 32768, 65536, -1],
     "graph_batch": [4, 2, 8],
     "split_spec": [3, 1, 2, 4, 6, -1],
     "prof_split": [2048, 512, 1024, 4096, 8192],

@@ -8,8 +8,10 @@
  *    halo index orders each halo's members by distance, equal distances in
  *    input order.  Haloes below NminPerHalo keep their order (AHF does not
  *    sort them).
- * 2. Unbinding: a persistent kernel, one workgroup per halo, haloes taken
- *    largest first from an atomic queue.  Per iteration:
+ * 2. Unbinding: persistent kernels by size, a wavefront or a workgroup per
+ *    halo that keeps the halo's members in registers, haloes taken largest
+ *    first from an atomic queue; the largest haloes over the chip (the split
+ *    path).  Per iteration:
  *      - dist_j, the mid-point terms of the integral of M(<r)/r^2 and their
  *        FP64 prefix sum Phi_j; Phi0 = Phi_{n-1} + n/dist_{n-1} (AHF's two
  *        passes add the same terms in the same order);
@@ -57,6 +59,9 @@ struct UnbindConst {
   int32_t minpart, no_vbulk;
   int32_t cut_before, unbind, cut_after, pad;
 };
+/* cut_before: the first rem_outsideRvir is made already (k_bin_forms), and the
+ * halo's record holds what it set, unless the record's pad says otherwise */
+#define CUT_DONE 2
 
 __device__ inline double wrap_s(double d)
 {
@@ -509,13 +514,14 @@ __device__ inline RecBound rec_bound(const UnbindConst &K, double Phi0, D4 asum,
  * bj holds the answer the sequential loop gives with that carry (the
  * dependence is strictly on earlier members, so any first guess settles).
  * Out: the chunk's bound totals (the same on every thread), whether a test
- * of the final evaluation was uncertain.  flag: two words of LDS, ev the
- * evaluation counter that alternates them.
+ * of the final evaluation was uncertain, and which of the thread's own were
+ * (bit i for member i).  flag: two words of LDS, ev the evaluation counter
+ * that alternates them.
  */
 template <int BS, int IPT>
 __device__ void settle_chunk(const UnbindConst &K, int64_t n, int64_t base, const double *dist, const double *phi,
                              const Staged &g, double Phi0, D4 cv, const RecBound &B, int bj[IPT], D4 *tot_out,
-                             int *unc_out, int *sweeps, D4 *sh4, int *sflag, int &ev)
+                             int *unc_out, uint32_t *unc_bits, int *sweeps, D4 *sh4, int *sflag, int &ev)
 {
   const int t = threadIdx.x;
   const int64_t j0 = base + (int64_t)t * IPT;
@@ -550,7 +556,8 @@ __device__ void settle_chunk(const UnbindConst &K, int64_t n, int64_t base, cons
     const D4 ex = blk_excl_scan4<BS>(run, &tot, sh4);
     /* the thread's own earlier members, summed again in the same order */
     D4 lex = {0, 0, 0, 0};
-    int chg = 0, unc = 0;
+    int chg = 0;
+    uint32_t unc = 0;
 #pragma unroll
     for (int i = 0; i < IPT; i++) {
       const int64_t j = j0 + i;
@@ -577,22 +584,211 @@ __device__ void settle_chunk(const UnbindConst &K, int64_t n, int64_t base, cons
                               e_vy * e_vy + e_vz * e_vz;
         const double tol = 4.0 * (e_vel2 + B.e_lim) + 1e-14 * (vel2 + lim);
         const double gap = fabs(vel2 - lim);
-        if (gap <= tol || gap <= K.band * lim) unc = 1;
+        if (gap <= tol || gap <= K.band * lim) unc |= 1u << i;
       }
       if (nb != bj[i]) { bj[i] = nb; chg = 1; }
     }
     if (t == 0) sflag[(ev + 1) & 1] = 0;
-    if (chg | unc) atomicOr(flag, chg | (unc << 1));
+    if (chg || unc) atomicOr(flag, chg | (unc ? 2 : 0));
     __syncthreads();
     const int f = *flag;
     ev++;
     if (!(f & 1)) {
       /* the statuses used were the final ones: so are the totals */
       *unc_out = f >> 1;
+      *unc_bits = unc;
       *tot_out = tot;
       return;
     }
   }
+}
+
+struct D3 {
+  double x, y, z;
+};
+
+/* one iteration in AHF's operation order, by one thread, over the halo's
+ * staged members (seed: the velocity of the bulk-velocity seed): st[j] as
+ * rem_unbound decides it; returns Phi0 */
+__device__ __noinline__ double replay_exact(const UnbindConst &K, int64_t n, D3 seed, const double *dist, uint8_t *st, const Staged &g)
+{
+  double I_now = 0, I_prev = 0, d_prev = 0, M_r = 0, P0 = 0, dd = 0;
+  for (int64_t j = 0; j < n; j++) {
+    M_r += 1.0;
+    dd = dist[j];
+    if (dd > MZERO) {
+      I_now = M_r / (dd * dd);
+      const double I_mid = (I_now + I_prev) / 2.;
+      P0 += I_mid * (dd - d_prev);
+    }
+    d_prev = dd;
+    I_prev = I_now;
+  }
+  P0 += M_r / dd;
+  double VX = seed.x, VY = seed.y, VZ = seed.z, M = 1.0, Phi = 0;
+  I_now = 0; I_prev = 0; d_prev = 0; M_r = 0;
+  for (int64_t j = 0; j < n; j++) {
+    M_r += 1.0;
+    const double dX = g.dx[j], dY = g.dy[j], dZ = g.dz[j];
+    dd = sqrt(dX * dX + dY * dY + dZ * dZ);
+    double v_esc2;
+    if (dd > MZERO) {
+      I_now = M_r / (dd * dd);
+      const double I_mid = (I_now + I_prev) / 2.;
+      Phi += I_mid * (dd - d_prev);
+      v_esc2 = (2 * fabs(Phi - P0) * K.phi_fac);
+    } else {
+      v_esc2 = 1e30;
+    }
+    const double fx = (double)g.vx[j], fy = (double)g.vy[j], fz = (double)g.vz[j];
+    const double dVX = (fx - VX / M) * K.v_fac + K.hubble * (dX) * K.r_fac;
+    const double dVY = (fy - VY / M) * K.v_fac + K.hubble * (dY) * K.r_fac;
+    const double dVZ = (fz - VZ / M) * K.v_fac + K.hubble * (dZ) * K.r_fac;
+    const double vel2 = dVX * dVX + dVY * dVY + dVZ * dVZ;
+    if (vel2 > K.v2_tune * v_esc2) {
+      st[j] = 0;
+    } else {
+      st[j] = 1;
+      M += 1.0;
+      VX += 1.0 * g.vx[j];
+      VY += 1.0 * g.vy[j];
+      VZ += 1.0 * g.vz[j];
+    }
+    I_prev = I_now;
+    d_prev = dd;
+  }
+  return P0;
+}
+
+/*
+ * One iteration's uncertain tests under AHF's rounding, by a workgroup of BS
+ * threads: st[j] bit 0 holds the status the certified tests found for member
+ * j, bit 1 that its test was uncertain.  AHF's running sums (the potential,
+ * the bulk velocity) are chains of FP64 additions of terms that are known for
+ * every member but the uncertain ones', whose statuses are assumed: so the
+ * other wavefronts lay the terms out in LDS and the first adds them up in list
+ * order, a lane a sum, and stops at the uncertain members only, to decide
+ * them with AHF's own values.  Two walks, as Phi0 is needed before the first
+ * test.  Should a decision differ from the status assumed, the later
+ * statuses rest on a wrong one, and thread 0 goes through the iteration
+ * member by member (replay_exact).  phi[j] of the uncertain members is
+ * overwritten.  Returns Phi0; bit 1 of every st[j] is cleared.
+ *
+ * Bound by the additions, about 5 ns a member and walk: an iteration of a
+ * halo of 1,815,480 members took 0.6 s member by member, 20 ms this way.
+ */
+template <int BS>
+__device__ __noinline__ double exact_iteration(const UnbindConst *Kp, int64_t n, double sx, double sy, double sz,
+                                               const double *dist, double *phi, uint8_t *st, const Staged *gp)
+{
+  constexpr int NW = BS / 64, W0 = NW > 1 ? 1 : 0; /* wavefronts from W0 on lay out */
+  constexpr int TB = 64 * (NW - W0);
+  __shared__ double s_t[2][3][TB + 2];
+  __shared__ uint64_t s_u[2][TB / 64], s_b[2][TB / 64];
+  __shared__ double s_p0;
+  __shared__ int s_bad;
+  const UnbindConst &K = *Kp;
+  const Staged g = *gp;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  if (t == 0) s_bad = 0;
+  const int64_t nb = (n + TB - 1) / TB;
+  for (int walk = 0; walk < 2; walk++) {
+    auto lay = [&](int64_t b, int buf) {
+      if (w < W0) return;
+      const int q = t - 64 * W0;
+      const int64_t j = b * TB + q;
+      double x0 = -0.0, x1 = -0.0, x2 = -0.0; /* leave any sum as it is */
+      const int s = j < n ? st[j] : 0;
+      if (j < n && walk == 0) {
+        const double dd = dist[j];
+        if (dd > MZERO) {
+          const double I_now = (double)(j + 1) / (dd * dd);
+          double I_prev = 0.0, d_prev = 0.0;
+          if (j > 0) {
+            d_prev = dist[j - 1];
+            int64_t k = j - 1; /* the last member before with a distance */
+            while (k >= 0 && !(dist[k] > MZERO)) k--;
+            if (k >= 0) I_prev = (double)(k + 1) / (dist[k] * dist[k]);
+          }
+          const double I_mid = (I_now + I_prev) / 2.;
+          x0 = I_mid * (dd - d_prev);
+        }
+      } else if (j < n && (s & 1)) {
+        x0 = (double)g.vx[j];
+        x1 = (double)g.vy[j];
+        x2 = (double)g.vz[j];
+      }
+      s_t[buf][0][q] = x0;
+      if (walk) {
+        s_t[buf][1][q] = x1;
+        s_t[buf][2][q] = x2;
+      }
+      const uint64_t um = __ballot((s >> 1) & 1), bm = __ballot(s & 1);
+      if (lane == 0) {
+        s_u[buf][q >> 6] = um;
+        s_b[buf][q >> 6] = bm;
+      }
+    };
+    const double P0 = walk ? s_p0 : 0.0;
+    const int row = walk && lane < 3 ? lane : 0;
+    double acc = !walk ? 0.0 : (lane == 1 ? sy : (lane == 2 ? sz : sx));
+    int64_t M = 1;
+    int bad = 0;
+    lay(0, 0);
+    __syncthreads();
+    for (int64_t b = 0; b < nb; b++) {
+      const int buf = (int)(b & 1);
+      if (b + 1 < nb) lay(b + 1, buf ^ 1);
+      if (w == 0 && !bad) {
+        for (int q = 0; q < TB; q += 64) {
+          const double *x = &s_t[buf][row][q];
+          const uint64_t um = s_u[buf][q >> 6], bm = s_b[buf][q >> 6];
+          if (um == 0ull) {
+#pragma unroll 16
+            for (int i = 0; i < 64; i++) acc += x[i];
+          } else {
+            for (int i = 0; i < 64; i++) {
+              const bool u = (um >> i) & 1ull;
+              const int64_t j = b * TB + q + i;
+              if (u && walk) {
+                const double VX = __shfl(acc, 0, 64), VY = __shfl(acc, 1, 64), VZ = __shfl(acc, 2, 64);
+                const double Md = (double)(M + __popcll(bm & ((1ull << i) - 1ull)));
+                const double dX = g.dx[j], dY = g.dy[j], dZ = g.dz[j];
+                const double v_esc2 = dist[j] > MZERO ? (2 * fabs(phi[j] - P0) * K.phi_fac) : 1e30;
+                const double dVX = ((double)g.vx[j] - VX / Md) * K.v_fac + K.hubble * (dX) * K.r_fac;
+                const double dVY = ((double)g.vy[j] - VY / Md) * K.v_fac + K.hubble * (dY) * K.r_fac;
+                const double dVZ = ((double)g.vz[j] - VZ / Md) * K.v_fac + K.hubble * (dZ) * K.r_fac;
+                const double vel2 = dVX * dVX + dVY * dVY + dVZ * dVZ;
+                const int bound = !(vel2 > K.v2_tune * v_esc2);
+                if (bound != (int)((bm >> i) & 1ull)) bad = 1;
+              }
+              acc += x[i];
+              if (u && !walk && lane == 0) phi[j] = acc;
+            }
+          }
+          M += __popcll(bm);
+        }
+      }
+      __syncthreads();
+    }
+    if (t == 0) {
+      if (!walk) s_p0 = acc + (double)n / dist[n - 1];
+      s_bad = bad;
+    }
+    __syncthreads();
+  }
+  const bool redo = s_bad != 0;
+  double P0 = s_p0;
+  if (redo) {
+    __syncthreads();
+    if (t == 0) s_p0 = replay_exact(K, n, D3{sx, sy, sz}, dist, st, g);
+    __syncthreads();
+    P0 = s_p0;
+  } else {
+    for (int64_t j = t; j < n; j += BS) st[j] &= 1;
+  }
+  __syncthreads();
+  return P0;
 }
 
 /*
@@ -602,9 +798,9 @@ __device__ void settle_chunk(const UnbindConst &K, int64_t n, int64_t base, cons
  * rounding factor gam of those parallel sums: st[j] = 1 for the members that
  * stay bound, as AHF's sequential loop decides them.  seed is the list
  * position of the bulk-velocity seed.  A member whose test the certified
- * rounding bound cannot settle sends the iteration to the exact sequential
- * replay (thread 0, in AHF's operation order), which also recomputes Phi0.
- * Returns 1 when it replayed.
+ * rounding bound cannot settle sends the iteration to exact_iteration, which
+ * also computes Phi0 as AHF does.  Returns 1 when it did.  phi: overwritten
+ * there.
  */
 /* where rec_eval starts when earlier members are settled already: member
  * j (a chunk boundary of the caller's), the totals before it, and whether
@@ -616,7 +812,7 @@ struct RecResume {
 };
 
 template <int BS, int IPT>
-__device__ int rec_eval(const UnbindConst &K, int64_t n, int64_t seed, const double *dist, const double *phi,
+__device__ int rec_eval(const UnbindConst &K, int64_t n, int64_t seed, const double *dist, double *phi,
                         uint8_t *st, Staged g, D4 asum, double gam, double *Phi0_io, int *sweeps,
                         const RecResume *resume = nullptr)
 {
@@ -624,7 +820,6 @@ __device__ int rec_eval(const UnbindConst &K, int64_t n, int64_t seed, const dou
   constexpr int64_t CH = (int64_t)BS * IPT;
   __shared__ D4 r_sh4[NW];
   __shared__ int sflag[2]; /* double-buffered: bit 0 a status changed, bit 1 a test was uncertain */
-  __shared__ double s_phi0;
   D4 *sh4 = r_sh4;
   const int t = threadIdx.x;
   if (t == 0) sflag[0] = sflag[1] = 0;
@@ -650,68 +845,20 @@ __device__ int rec_eval(const UnbindConst &K, int64_t n, int64_t seed, const dou
     for (int i = 0; i < IPT; i++) bj[i] = j0 + i < n ? 1 : 0;
     D4 tot;
     int unc = 0;
-    settle_chunk<BS, IPT>(K, n, base, dist, phi, g, Phi0, cv, B, bj, &tot, &unc, sweeps, sh4, sflag, ev);
+    uint32_t ub = 0;
+    settle_chunk<BS, IPT>(K, n, base, dist, phi, g, Phi0, cv, B, bj, &tot, &unc, &ub, sweeps, sh4, sflag, ev);
     uncertain |= unc;
     cv.x += tot.x; cv.y += tot.y; cv.z += tot.z; cv.m += tot.m;
 #pragma unroll
     for (int i = 0; i < IPT; i++)
-      if (j0 + i < n) st[j0 + i] = (uint8_t)bj[i];
+      if (j0 + i < n) st[j0 + i] = (uint8_t)(bj[i] | ((ub >> i) & 1u) << 1);
   }
   __syncthreads();
-  /* exact replay of this iteration where rounding could decide (thread 0) */
+  /* where rounding could decide: those tests under AHF's own rounding */
   int replayed = 0;
   if (uncertain) {
     replayed = 1;
-    if (t == 0) {
-      double I_now = 0, I_prev = 0, d_prev = 0, M_r = 0, P0 = 0, dd = 0;
-      for (int64_t j = 0; j < n; j++) {
-        M_r += 1.0;
-        dd = dist[j];
-        if (dd > MZERO) {
-          I_now = M_r / (dd * dd);
-          const double I_mid = (I_now + I_prev) / 2.;
-          P0 += I_mid * (dd - d_prev);
-        }
-        d_prev = dd;
-        I_prev = I_now;
-      }
-      P0 += M_r / dd;
-      s_phi0 = P0;
-      double VX = sx, VY = sy, VZ = sz, M = 1.0, Phi = 0;
-      I_now = 0; I_prev = 0; d_prev = 0; M_r = 0;
-      for (int64_t j = 0; j < n; j++) {
-        M_r += 1.0;
-        const double dX = g.dx[j], dY = g.dy[j], dZ = g.dz[j];
-        dd = sqrt(dX * dX + dY * dY + dZ * dZ);
-        double v_esc2;
-        if (dd > MZERO) {
-          I_now = M_r / (dd * dd);
-          const double I_mid = (I_now + I_prev) / 2.;
-          Phi += I_mid * (dd - d_prev);
-          v_esc2 = (2 * fabs(Phi - P0) * K.phi_fac);
-        } else {
-          v_esc2 = 1e30;
-        }
-        const double fx = (double)g.vx[j], fy = (double)g.vy[j], fz = (double)g.vz[j];
-        const double dVX = (fx - VX / M) * K.v_fac + K.hubble * (dX) * K.r_fac;
-        const double dVY = (fy - VY / M) * K.v_fac + K.hubble * (dY) * K.r_fac;
-        const double dVZ = (fz - VZ / M) * K.v_fac + K.hubble * (dZ) * K.r_fac;
-        const double vel2 = dVX * dVX + dVY * dVY + dVZ * dVZ;
-        if (vel2 > K.v2_tune * v_esc2) {
-          st[j] = 0;
-        } else {
-          st[j] = 1;
-          M += 1.0;
-          VX += 1.0 * g.vx[j];
-          VY += 1.0 * g.vy[j];
-          VZ += 1.0 * g.vz[j];
-        }
-        I_prev = I_now;
-        d_prev = dd;
-      }
-    }
-    __syncthreads();
-    Phi0 = s_phi0;
+    Phi0 = exact_iteration<BS>(&K, n, sx, sy, sz, dist, phi, st, &g);
   }
   *Phi0_io = Phi0;
   __syncthreads();
@@ -739,7 +886,12 @@ __device__ void unbind_halo(const UnbindConst &K, int64_t n0, int64_t seed0, uin
   int64_t pit = 0;
   /* rem_outsideRvir(halo, 0): returns below minpart, else cuts and clears
    * Phi0 (:3696, :3864-3871) */
-  if (K.cut_before && n >= K.minpart) {
+  if (K.cut_before == CUT_DONE && !out->pad) {
+    M_vir = out->M_vir;
+    R_vir = out->R_vir;
+    ovdens = out->ovdens;
+    set = out->set;
+  } else if (K.cut_before && n >= K.minpart) {
     n = rvir_cut<BS>(K, n, cur, cen, pv, &M_vir, &R_vir, &ovdens);
     Phi0 = 0.0;
     set = AHFGPU_SET_MVIR | AHFGPU_SET_RVIR | AHFGPU_SET_PHI0 | AHFGPU_SET_OVDENS;
@@ -895,7 +1047,498 @@ __device__ void unbind_halo(const UnbindConst &K, int64_t n0, int64_t seed0, uin
     out->set = set;
     out->particle_iterations = pit;
     out->sweeps = sweeps;
+    out->pad = 0;
   }
+}
+
+#define AHF_UNBIND_IPT 4
+
+/*
+ * The unbinding of one halo of at most BS*IPT members by one workgroup of BS
+ * threads that keeps the halo in registers: thread t holds the list's members
+ * [t*IPT, (t+1)*IPT) for the whole unbinding, each with its distance, Hubble
+ * term and velocity, and a bit that says whether it is still bound.  The
+ * members are gathered once; an iteration reads and writes no memory, a
+ * removed member clears its bit (members only leave, so the ranks among the
+ * bits are the list's positions), and the list is written once at the end,
+ * in place.
+ *
+ * The work of an iteration is the chunked form's (unbind_halo), with the
+ * whole halo as one chunk.  That form gathers, stages, re-reads and compacts
+ * through memory in every iteration and pass and is bound by those round
+ * trips: 20,000 haloes' tiers of 64, 256 and 512 threads took 0.55, 0.90 and
+ * 0.63 ms.  Here an iteration is bound by the latency of its block scans and
+ * of the FP64 chain of a thread's IPT members.
+ */
+template <int NW>
+struct ResShared {
+  D4 asum;
+  D4 sum4[NW], tot[2][NW];
+  double sum[NW], last[NW];
+  double fx, fy, fz; /* a member handed to every thread */
+  double M, R, od;
+  int32_t cnt[NW], has[NW];
+  int32_t flag[NW], moved[2][NW];
+  unsigned long long first;
+};
+
+__device__ __forceinline__ D4 add4(D4 a, D4 b) { return D4{a.x + b.x, a.y + b.y, a.z + b.z, a.m + b.m}; }
+/* the last lane's value */
+__device__ __forceinline__ D4 res_top4(D4 a)
+{
+  return D4{__shfl(a.x, 63, 64), __shfl(a.y, 63, 64), __shfl(a.z, 63, 64), __shfl(a.m, 63, 64)};
+}
+
+/* over the workgroup's threads: exclusive scan of D4 and its total */
+template <int BS>
+__device__ __forceinline__ D4 res_scan4(D4 v, D4 *tot, ResShared<BS / 64> &S)
+{
+  if constexpr (BS == 64) {
+    D4 inc, ex;
+    wave_scan4_dpp(v, &inc, &ex);
+    *tot = res_top4(inc);
+    return ex;
+  } else {
+    return blk_excl_scan4<BS>(v, tot, S.sum4);
+  }
+}
+
+template <int BS>
+__device__ __forceinline__ double res_scan(double v, double *tot, ResShared<BS / 64> &S)
+{
+  if constexpr (BS == 64) {
+    double a = v;
+    a += dpp_d<0x111, 0xf>(a); /* as wave_scan4_dpp */
+    a += dpp_d<0x112, 0xf>(a);
+    a += dpp_d<0x114, 0xf>(a);
+    a += dpp_d<0x118, 0xf>(a);
+    a += dpp_d<0x142, 0xa>(a);
+    a += dpp_d<0x143, 0xc>(a);
+    *tot = __shfl(a, 63, 64);
+    return dpp_d<0x138, 0xf>(a);
+  } else {
+    return blk_excl_scan<BS, double>(v, tot, S.sum);
+  }
+}
+
+/* 1 when v is not 0 on some thread of the workgroup */
+template <int BS>
+__device__ __forceinline__ int res_or(int v, ResShared<BS / 64> &S)
+{
+  const int f = __ballot(v != 0) ? 1 : 0;
+  if constexpr (BS == 64) return f;
+  if ((threadIdx.x & 63) == 0) S.flag[threadIdx.x >> 6] = f;
+  __syncthreads();
+  int r = 0;
+#pragma unroll
+  for (int k = 0; k < BS / 64; k++) r |= S.flag[k];
+  __syncthreads();
+  return r;
+}
+
+/* positions in the list of the members still bound: the thread's first one's
+ * (r0), their number (n), the distance of the one before the thread's first
+ * (dprev, 0 when there is none) and of the list's last (dlast) */
+template <int BS, int IPT>
+__device__ __forceinline__ void res_ranks(uint32_t alive, const double d[IPT], int *r0, int *n, double *dprev,
+                                          double *dlast, ResShared<BS / 64> &S)
+{
+  constexpr int NW = BS / 64;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = __popc(alive);
+  double ld = 0.0;
+#pragma unroll
+  for (int i = 0; i < IPT; i++)
+    if ((alive >> i) & 1u) ld = d[i];
+  int inc = c;
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x111, 0xf, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x112, 0xf, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x114, 0xf, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x118, 0xf, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);
+  const uint64_t has = __ballot(c > 0), below = has & ((1ull << lane) - 1ull);
+  const double wprev = __shfl(ld, below ? 63 - __builtin_clzll(below) : 0, 64);
+  const double wlast = __shfl(ld, has ? 63 - __builtin_clzll(has) : 0, 64);
+  const int wtot = __shfl(inc, 63, 64);
+  if constexpr (BS == 64) {
+    *r0 = inc - c;
+    *n = wtot;
+    *dprev = below ? wprev : 0.0;
+    *dlast = has ? wlast : 0.0;
+  } else {
+    if (lane == 0) {
+      S.cnt[w] = wtot;
+      S.last[w] = wlast;
+      S.has[w] = has != 0;
+    }
+    __syncthreads();
+    int base = 0, tot = 0;
+    double dp = 0.0, dl = 0.0;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+      const int ck = S.cnt[k];
+      if (k < w) {
+        base += ck;
+        if (S.has[k]) dp = S.last[k];
+      }
+      tot += ck;
+      if (S.has[k]) dl = S.last[k];
+    }
+    __syncthreads();
+    *r0 = base + inc - c;
+    *n = tot;
+    *dprev = below ? wprev : dp;
+    *dlast = dl;
+  }
+}
+
+/* rem_outsideRvir over the members still bound (rvir_cut's rule): clears the
+ * bits after the first member whose sphere is below ovlim; M_vir, R_vir and
+ * ovdens of the last one kept on every thread.  r0, n: res_ranks' */
+template <int BS, int IPT>
+__device__ __forceinline__ void res_cut(const UnbindConst &K, uint32_t *alive, const double d[IPT], int r0, int n,
+                                        double *M, double *R, double *od, ResShared<BS / 64> &S)
+{
+  if (threadIdx.x == 0) S.first = ~0ull;
+  __syncthreads();
+  int first = INT32_MAX, r = r0;
+  double o[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    o[i] = 0.0;
+    if (!((*alive >> i) & 1u)) continue;
+    const double V = 4. * PI_AHF / 3. * (d[i] * d[i] * d[i]);
+    o[i] = (double)(r + 1) / V * K.rho_fac / K.rho_vir;
+    if (!(o[i] >= K.ovlim) && r < first) first = r;
+    r++;
+  }
+  if (first != INT32_MAX) atomicMin(&S.first, (unsigned long long)first);
+  __syncthreads();
+  const int kept = S.first != ~0ull ? (int)S.first + 1 : n;
+  r = r0;
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    if (!((*alive >> i) & 1u)) continue;
+    if (r == kept - 1) {
+      S.M = (double)kept;
+      S.R = d[i];
+      S.od = o[i];
+    }
+    if (r >= kept) *alive &= ~(1u << i);
+    r++;
+  }
+  __syncthreads();
+  *M = S.M;
+  *R = S.R;
+  *od = S.od;
+  __syncthreads();
+}
+
+template <int BS, int IPT>
+__device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0, int64_t seed0, uint32_t *a, double *dist,
+                                                double *phi, uint8_t *st, Staged g, const double cen[3],
+                                                const float4 *__restrict__ pv, HaloOut *out)
+{
+  constexpr int NW = BS / 64;
+  __shared__ ResShared<NW> S;
+  __shared__ double s_h[3][IPT][BS]; /* the Hubble terms */
+  const int t = threadIdx.x, j0 = t * IPT;
+  double d[IPT], lm[IPT];
+  float vx[IPT], vy[IPT], vz[IPT];
+  uint32_t alive = 0;
+  D4 av = {0, 0, 0, 0};
+  uint32_t p[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; i++) p[i] = j0 + i < n0 ? a[j0 + i] : 0u;
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    d[i] = 0.0;
+    vx[i] = vy[i] = vz[i] = 0.0f;
+    if (j0 + i >= n0) continue;
+    const float4 q0 = pv[2 * (size_t)p[i]], q1 = pv[2 * (size_t)p[i] + 1];
+    const double dX = wrap_s((double)q0.x - cen[0]), dY = wrap_s((double)q0.y - cen[1]), dZ = wrap_s((double)q0.z - cen[2]);
+    d[i] = sqrt(dX * dX + dY * dY + dZ * dZ);
+    s_h[0][i][t] = K.hubble * dX * K.r_fac;
+    s_h[1][i][t] = K.hubble * dY * K.r_fac;
+    s_h[2][i][t] = K.hubble * dZ * K.r_fac;
+    vx[i] = q0.w;
+    vy[i] = q1.x;
+    vz[i] = q1.y;
+    alive |= 1u << i;
+    av.x += fabs((double)q0.w);
+    av.y += fabs((double)q1.x);
+    av.z += fabs((double)q1.y);
+    if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0); /* the loads of four members in flight */
+  }
+  /* the sums of |v| that bound the rounding of the bulk-velocity sums: over
+   * the whole list, so no smaller than over the members still bound */
+  {
+    D4 asum;
+    (void)res_scan4<BS>(av, &asum, S);
+    if (t == 0) S.asum = asum;
+  }
+  int n = (int)n0, r0 = 0, niter = 0, replays = 0, rvir_set = 0, sweeps = 0, set = 0;
+  double dprev, dlast;
+  double R_vir = 0.0, Phi0 = 0.0, M_vir = 0.0, ovdens = 0.0;
+  int64_t pit = 0;
+  res_ranks<BS, IPT>(alive, d, &r0, &n, &dprev, &dlast, S);
+  if (K.cut_before == CUT_DONE) {
+    M_vir = out->M_vir;
+    R_vir = out->R_vir;
+    ovdens = out->ovdens;
+    set = out->set;
+  } else if (K.cut_before && n >= K.minpart) {
+    res_cut<BS, IPT>(K, &alive, d, r0, n, &M_vir, &R_vir, &ovdens, S);
+    Phi0 = 0.0;
+    set = AHFGPU_SET_MVIR | AHFGPU_SET_RVIR | AHFGPU_SET_PHI0 | AHFGPU_SET_OVDENS;
+    res_ranks<BS, IPT>(alive, d, &r0, &n, &dprev, &dlast, S);
+  }
+  const bool unbind = K.unbind && n >= K.minpart;
+  if (unbind) {
+    R_vir = 0.0;
+    set = (set | AHFGPU_SET_MVIR | AHFGPU_SET_PHI0) & ~AHFGPU_SET_RVIR;
+  }
+  int nremove = unbind ? 4 : 0;
+  while (nremove > 3) {
+    niter++;
+    pit += n;
+    /* mid-point terms and their prefix sum Phi_j (kept in lm) */
+    double run = 0.0;
+    {
+      int r = r0; /* position of the next member; members before it */
+      double dp = dprev, Ip = r > 0 && dp > MZERO ? (double)r / (dp * dp) : 0.0;
+#pragma unroll
+      for (int i = 0; i < IPT; i++) {
+        lm[i] = 0.0;
+        if (!((alive >> i) & 1u)) continue;
+        double I_now = 0.0;
+        if (d[i] > MZERO) {
+          I_now = (double)(r + 1) / (d[i] * d[i]);
+          const double I_mid = (I_now + Ip) / 2.;
+          run += I_mid * (d[i] - dp);
+        }
+        lm[i] = run;
+        dp = d[i];
+        Ip = I_now;
+        r++;
+        if (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    double tot1;
+    const double ex1 = res_scan<BS>(run, &tot1, S);
+    Phi0 = tot1 + (double)n / dlast;
+    /* the limits v2_tune*v_esc2, with no limit inside MACHINE_ZERO */
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      lm[i] = d[i] > MZERO ? K.v2_tune * (2 * fabs((ex1 + lm[i]) - Phi0) * K.phi_fac) : -1.0;
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    /* the bulk-velocity seed: the list's position seed0 at first, then the
+     * first member still bound */
+    {
+      const int sp = niter == 1 ? (int)seed0 : 0;
+      int r = r0;
+#pragma unroll
+      for (int i = 0; i < IPT; i++) {
+        if (!((alive >> i) & 1u)) continue;
+        if (r == sp) {
+          S.fx = (double)vx[i];
+          S.fy = (double)vy[i];
+          S.fz = (double)vz[i];
+        }
+        r++;
+      }
+      __syncthreads();
+    }
+    const D3 seed = {S.fx, S.fy, S.fz};
+    const double Nd = (double)n + 8.0, U = 1.1102230246251565e-16;
+    const RecBound B = rec_bound(K, Phi0, S.asum, Nd * U / (1.0 - Nd * U));
+    /*
+     * The sequential recurrence (settle_chunk's tests).  A thread takes its
+     * members in order with the bulk velocity that it has just changed; a
+     * wavefront evaluates its members again, with the totals of its lower
+     * lanes' last statuses, until none changes; the wavefronts then hand up
+     * their totals, until no total changes.  Every evaluation settles at
+     * least one thread more and every hand-over one wavefront more, and what
+     * no longer changes is the sequential answer.  (Whole-list sweeps with
+     * the statuses of the sweep before settle one member at a time where
+     * statuses near the centre hang on each other: 1.9 ms for the haloes of
+     * 513 to 2048 members of 20,000, where this takes 0.11.)
+     * V/M as V times 1/M: within 1.5 units of rounding of the quotient, which
+     * the bound's fifth gam*sum|v| (at least 28 units) has room for.
+     */
+    uint32_t bj = alive, ub = 0;
+    const int w = t >> 6;
+    D4 base = {seed.x, seed.y, seed.z, 1.0}, mine = {0, 0, 0, 0};
+    auto sums = [&]() {
+      /* the velocities are converted in every evaluation: kept as doubles
+       * from one to the next (the compiler would) they do not fit */
+#pragma unroll
+      for (int i = 0; i < IPT; i++) asm volatile("" : "+v"(vx[i]), "+v"(vy[i]), "+v"(vz[i]));
+      D4 sum = {0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < IPT; i++)
+        if ((bj >> i) & 1u) {
+          sum.x += (double)vx[i];
+          sum.y += (double)vy[i];
+          sum.z += (double)vz[i];
+          sum.m += 1.0;
+        }
+      return sum;
+    };
+    /* the wavefronts below (round 0: all members bound) */
+    if constexpr (NW > 1) {
+      D4 inc, ex;
+      wave_scan4_dpp(sums(), &inc, &ex);
+      mine = res_top4(inc);
+      if ((t & 63) == 0) S.tot[0][w] = mine;
+      __syncthreads();
+      for (int k = 0; k < w; k++) base = add4(base, S.tot[0][k]);
+    }
+    for (int round = 1;; round++) {
+      D4 inc, ex;
+      for (;;) {
+        sweeps++;
+        wave_scan4_dpp(sums(), &inc, &ex);
+        D4 V = add4(base, ex);
+        uint32_t nb = 0;
+        ub = 0;
+#pragma unroll
+        for (int i = 0; i < IPT; i++) {
+          if (!((alive >> i) & 1u)) continue;
+          const double fx = (double)vx[i], fy = (double)vy[i], fz = (double)vz[i];
+          const double rM = 1.0 / V.m;
+          const double dVX = (fx - V.x * rM) * K.v_fac + s_h[0][i][t];
+          const double dVY = (fy - V.y * rM) * K.v_fac + s_h[1][i][t];
+          const double dVZ = (fz - V.z * rM) * K.v_fac + s_h[2][i][t];
+          const double vel2 = dVX * dVX + dVY * dVY + dVZ * dVZ;
+          const double lim = lm[i] >= 0.0 ? lm[i] : K.v2_tune * 1e30;
+          if (lm[i] >= 0.0) {
+            const double e_vx = B.cvx * rM, e_vy = B.cvy * rM, e_vz = B.cvz * rM;
+            const double e_vel2 = 2.0 * (fabs(dVX) * e_vx + fabs(dVY) * e_vy + fabs(dVZ) * e_vz) + e_vx * e_vx +
+                                  e_vy * e_vy + e_vz * e_vz;
+            const double tol = 4.0 * (e_vel2 + B.e_lim) + 1e-14 * (vel2 + lim);
+            const double gap = fabs(vel2 - lim);
+            if (gap <= tol || gap <= K.band * lim) ub |= 1u << i;
+          }
+          if (!(vel2 > lim)) {
+            nb |= 1u << i;
+            V.x += fx;
+            V.y += fy;
+            V.z += fz;
+            V.m += 1.0;
+          }
+          /* one member after the other: interleaved by the scheduler, their
+           * temporaries do not fit beside the members */
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const uint64_t chg = __ballot(nb != bj);
+        bj = nb;
+        if (chg == 0ull) break;
+      }
+      if constexpr (NW == 1) break;
+      const D4 now = res_top4(inc);
+      const int moved = now.x != mine.x || now.y != mine.y || now.z != mine.z || now.m != mine.m;
+      mine = now;
+      if ((t & 63) == 0) {
+        S.tot[round & 1][w] = now;
+        S.moved[round & 1][w] = moved;
+      }
+      __syncthreads();
+      int any = 0;
+      for (int k = 0; k + 1 < NW; k++) any |= S.moved[round & 1][k];
+      if (!any) break;
+      base = D4{seed.x, seed.y, seed.z, 1.0};
+      for (int k = 0; k < w; k++) base = add4(base, S.tot[round & 1][k]);
+    }
+    if (res_or<BS>(ub != 0, S)) {
+      /* the uncertain tests, over the members staged in list order */
+      replays++;
+      int r = r0;
+#pragma unroll
+      for (int i = 0; i < IPT; i++) {
+        if (!((alive >> i) & 1u)) continue;
+        const float4 q0 = pv[2 * (size_t)a[j0 + i]];
+        dist[r] = d[i];
+        g.dx[r] = wrap_s((double)q0.x - cen[0]);
+        g.dy[r] = wrap_s((double)q0.y - cen[1]);
+        g.dz[r] = wrap_s((double)q0.z - cen[2]);
+        g.vx[r] = vx[i];
+        g.vy[r] = vy[i];
+        g.vz[r] = vz[i];
+        st[r] = (uint8_t)(((bj >> i) & 1u) | ((ub >> i) & 1u) << 1);
+        r++;
+      }
+      __syncthreads();
+      Phi0 = exact_iteration<BS>(&K, n, seed.x, seed.y, seed.z, dist, phi, st, &g);
+      bj = 0;
+      r = r0;
+#pragma unroll
+      for (int i = 0; i < IPT; i++) {
+        if (!((alive >> i) & 1u)) continue;
+        if (st[r]) bj |= 1u << i;
+        r++;
+      }
+      __syncthreads();
+    }
+    alive = bj;
+    const int before = n;
+    res_ranks<BS, IPT>(alive, d, &r0, &n, &dprev, &dlast, S);
+    nremove = before - n;
+    M_vir = (double)n;
+    if (n > 0) {
+      R_vir = dlast;
+      rvir_set = 1;
+    }
+    if ((double)n < (double)K.minpart) break;
+  }
+  if (rvir_set) set |= AHFGPU_SET_RVIR;
+  if (K.cut_after && n >= K.minpart) {
+    res_cut<BS, IPT>(K, &alive, d, r0, n, &M_vir, &R_vir, &ovdens, S);
+    set |= AHFGPU_SET_MVIR | AHFGPU_SET_RVIR | AHFGPU_SET_OVDENS;
+    res_ranks<BS, IPT>(alive, d, &r0, &n, &dprev, &dlast, S);
+  }
+  /* the list in place: every thread has read its members before any writes */
+#pragma unroll
+  for (int i = 0; i < IPT; i++) p[i] = (alive >> i) & 1u ? a[j0 + i] : 0u;
+  __syncthreads();
+  {
+    int r = r0;
+#pragma unroll
+    for (int i = 0; i < IPT; i++)
+      if ((alive >> i) & 1u) a[r++] = p[i];
+  }
+  if (t == 0) {
+    out->npart = n;
+    out->M_vir = M_vir;
+    out->R_vir = R_vir;
+    out->Phi0 = Phi0;
+    out->ovdens = ovdens;
+    out->niter = niter;
+    out->replays = replays;
+    out->in_b = 0;
+    out->set = set;
+    out->particle_iterations = pit;
+    out->sweeps = sweeps;
+    out->pad = 0;
+  }
+}
+
+/* one halo on a workgroup of BS threads: in registers, IPT members a thread
+ * (UF_EITHER: 2 or 8, by the halo's size), or (IPT 0) in chunks through
+ * memory */
+#define UF_EITHER 28
+template <int BS, int IPT>
+__device__ __forceinline__ void unbind_form(const UnbindConst &K, int64_t n, int64_t seed0, uint32_t *a, uint32_t *b,
+                                            double *dist, double *phi, uint8_t *st, Staged g, const double cen[3],
+                                            const float4 *__restrict__ pv, HaloOut *out)
+{
+  if constexpr (IPT == UF_EITHER) {
+    if (n <= 2 * BS) unbind_resident<BS, 2>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
+    else unbind_resident<BS, 8>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
+  } else if constexpr (IPT > 0) unbind_resident<BS, IPT>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
+  else unbind_halo<BS, AHF_UNBIND_IPT>(K, n, seed0, a, b, dist, phi, st, g, cen, pv, out);
 }
 
 /* the first iteration's seed of every halo (:3441-3470): the median |v|^2
@@ -938,19 +1581,56 @@ static inline unsigned seed_blocks(int64_t nh)
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nh, (int64_t)1 << 20));
 }
 
-/* haloes of at least this many members go to 512-thread workgroups */
-#define AHF_BIG_HALO 2048
-#define AHF_WAVE_HALO 512 /* haloes below this many members: one wavefront each */
+/*
+ * The forms of the unbinding by size, largest first: in chunks through memory
+ * (512 threads) what no workgroup holds, then in registers on 512 threads,
+ * 256 threads and one wavefront, 8 members a thread, and on one wavefront
+ * with 2 (twice as many of them resident).  The schedule's big_halo and
+ * wave_halo move the lines between the register forms below that.  The
+ * kernels are bound by the serial chain of the longest halo's iterations, not
+ * by memory: in registers an iteration has no pass over memory and one barrier
+ * a hand-over.  Against chunks for every size (unbinding alone): 2,000 lists of
+ * 20 to 100,000 members 0.78 -> 0.69 ms, 20,000 lists 1.9 -> 1.4 ms, and 16
+ * lists end to end 213 -> 192 us.
+ */
+enum { UF_CHUNK = 0, UF_BIG, UF_MID, UF_WAVE, UF_SMALL, UF_FORMS };
 #define AHF_BIG_BLOCK 512
-#define AHF_UNBIND_IPT 4
+#define AHF_BIG_MOST 4096
+#define AHF_MID_MOST 2048
+#define AHF_WAVE_MOST 512
+#define AHF_SMALL_MOST 128
+
+/* the least members of form f (0 for the last) */
+static inline int64_t uf_least(const ahfgpu_ctx *c, int f)
+{
+  const int64_t mid1 = c->big_halo > 0 ? std::min<int64_t>(c->big_halo, AHF_MID_MOST + 1) : AHF_MID_MOST + 1;
+  const int64_t wave1 = c->wave_halo > 0 ? std::min<int64_t>(c->wave_halo, AHF_WAVE_MOST + 1) : AHF_WAVE_MOST + 1;
+  switch (f) {
+  case UF_CHUNK: return AHF_BIG_MOST + 1;
+  case UF_BIG: return mid1;
+  case UF_MID: return std::min(mid1, wave1);
+  case UF_WAVE: return std::min<int64_t>(std::min(mid1, wave1), AHF_SMALL_MOST + 1);
+  default: return 0;
+  }
+}
+
+/* one launch for both wavefront forms: as many haloes as are resident at once
+ * in it; behind the cut, which leaves few members of most, twice as many */
+static inline bool uf_either(bool binned, int64_t haloes, int cu) { return haloes <= (int64_t)cu * (binned ? 16 : 8); }
+
+/* wavefronts a SIMD for which the registers are held down: 256 of them hold
+ * 8 members and an evaluation's temporaries, 128 hold 2 */
+#define AHF_UNBIND_WAVES(IPT) ((IPT) == 2 ? 4 : 2)
 
 /* persistent form: workgroups take haloes order[q0..q1) from the queue
  * (largest first) */
-template <int BS>
-__device__ void unbind_queue(const UnbindConst &K, const int64_t *__restrict__ off, const int32_t *__restrict__ order,
-                             int64_t q0, int64_t q1, int32_t *__restrict__ next, const int64_t *__restrict__ seed,
-                             uint32_t *a, uint32_t *b, double *dist, double *phi, uint8_t *st, Staged g,
-                             const double *__restrict__ cen, const float4 *__restrict__ pv, HaloOut *__restrict__ out)
+template <int BS, int IPT>
+__device__ __forceinline__ void unbind_queue(const UnbindConst &K, const int64_t *__restrict__ off,
+                                             const int32_t *__restrict__ order, int64_t q0, int64_t q1,
+                                             int32_t *__restrict__ next, const int64_t *__restrict__ seed, uint32_t *a,
+                                             uint32_t *b, double *dist, double *phi, uint8_t *st, Staged g,
+                                             const double *__restrict__ cen, const float4 *__restrict__ pv,
+                                             HaloOut *__restrict__ out)
 {
   __shared__ int64_t sh_h;
   for (;;) {
@@ -962,53 +1642,138 @@ __device__ void unbind_queue(const UnbindConst &K, const int64_t *__restrict__ o
     const int64_t h = sh_h;
     __syncthreads();
     if (h < 0) return;
-    const int64_t o = off[h], n = off[h + 1] - o;
+    const int64_t o = off[h], n = K.cut_before == CUT_DONE ? out[h].npart : off[h + 1] - o;
     const double c3[3] = {cen[3 * h], cen[3 * h + 1], cen[3 * h + 2]};
     const Staged go = {g.dx + o, g.dy + o, g.dz + o, g.vx + o, g.vy + o, g.vz + o};
-    unbind_halo<BS, AHF_UNBIND_IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
+    unbind_form<BS, IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
     __syncthreads();
   }
 }
 
-template <int BS>
-__global__ void __launch_bounds__(BS) k_unbind_batched(UnbindConst K, const int64_t *__restrict__ off,
-                                                       const int32_t *__restrict__ order, int64_t q0, int64_t q1,
-                                                       int32_t *__restrict__ next, const int64_t *__restrict__ seed,
-                                                       uint32_t *a, uint32_t *b, double *dist, double *phi,
-                                                       uint8_t *st, Staged g,
-                                                       const double *__restrict__ cen, const float4 *__restrict__ pv, HaloOut *__restrict__ out)
+template <int BS, int IPT>
+__global__ void __launch_bounds__(BS, AHF_UNBIND_WAVES(IPT))
+    k_unbind(UnbindConst K, const int64_t *__restrict__ off, const int32_t *__restrict__ order, int64_t q0, int64_t q1,
+             int32_t *__restrict__ next, const int64_t *__restrict__ seed, uint32_t *a, uint32_t *b, double *dist,
+             double *phi, uint8_t *st, Staged g, const double *__restrict__ cen, const float4 *__restrict__ pv,
+             HaloOut *__restrict__ out)
 {
-  unbind_queue<BS>(K, off, order, q0, q1, next, seed, a, b, dist, phi, st, g, cen, pv, out);
+  unbind_queue<BS, IPT>(K, off, order, q0, q1, next, seed, a, b, dist, phi, st, g, cen, pv, out);
 }
 
-/* the same with the queue range read from the device: order[qb[tier] ..
- * qb[tier + 1]) */
-template <int BS>
-__global__ void __launch_bounds__(BS) k_unbind_batched_dq(UnbindConst K, const int64_t *__restrict__ off,
-                                                          const int32_t *__restrict__ order,
-                                                          const int64_t *__restrict__ qb, int tier,
-                                                          int32_t *__restrict__ next, const int64_t *__restrict__ seed,
-                                                          uint32_t *a, uint32_t *b, double *dist, double *phi,
-                                                          uint8_t *st, Staged g, const double *__restrict__ cen,
-                                                          const float4 *__restrict__ pv,
-                                                          HaloOut *__restrict__ out)
+/* the same over a list made on the device (k_bin_forms) */
+template <int BS, int IPT>
+__global__ void __launch_bounds__(BS, AHF_UNBIND_WAVES(IPT))
+    k_unbind_dq(UnbindConst K, const int64_t *__restrict__ off, const int32_t *__restrict__ list,
+                const int32_t *__restrict__ cnt, int32_t *__restrict__ next, const int64_t *__restrict__ seed, uint32_t *a,
+                uint32_t *b, double *dist, double *phi, uint8_t *st, Staged g, const double *__restrict__ cen,
+                const float4 *__restrict__ pv, HaloOut *__restrict__ out)
 {
-  unbind_queue<BS>(K, off, order, qb[tier], qb[tier + 1], next, seed, a, b, dist, phi, st, g, cen, pv, out);
+  unbind_queue<BS, IPT>(K, off, list, 0, *cnt, next, seed, a, b, dist, phi, st, g, cen, pv, out);
+}
+
+struct FormLeast {
+  int64_t v[UF_FORMS];
+};
+
+/* rem_outsideRvir's cut (rvir_cut's rule) of the first n >= 1 members of list
+ * l by one workgroup with one barrier a step; M, R and od on every thread.
+ * The members' records lie anywhere in memory and most are beyond the cut: the
+ * first step takes one member a thread, the others four. */
+template <int PER>
+__device__ __forceinline__ int64_t group_cut_step(const UnbindConst &K, int64_t base, int64_t n, const uint32_t *l,
+                                                  const double cen[3], const float4 *__restrict__ pv, int64_t *s_first)
+{
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t j0 = base + (int64_t)wave * 64 * PER + lane;
+  uint32_t p[PER];
+  bool low[PER];
+#pragma unroll
+  for (int i = 0; i < PER; i++) p[i] = j0 + 64 * i < n ? l[j0 + 64 * i] : 0u;
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    double r;
+    low[i] = j0 + 64 * i < n && !(sphere_ovdens(K, j0 + 64 * i, p[i], cen, pv, &r) >= K.ovlim);
+  }
+  int64_t first = n;
+#pragma unroll
+  for (int i = PER - 1; i >= 0; i--) {
+    const uint64_t f = __ballot(low[i]);
+    if (f) first = j0 - lane + 64 * i + __builtin_ctzll(f) + 1;
+  }
+  if (lane == 0) s_first[wave] = first;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < AHF_BLOCK / 64; w++) first = min(first, s_first[w]);
+  return first;
+}
+
+__device__ __forceinline__ int64_t group_cut(const UnbindConst &K, int64_t n, const uint32_t *l, const double cen[3],
+                                             const float4 *__restrict__ pv, double *M, double *R, double *od)
+{
+  __shared__ int64_t s_first[2][AHF_BLOCK / 64];
+  int64_t kept = group_cut_step<1>(K, 0, n, l, cen, pv, s_first[0]);
+  int buf = 1;
+  for (int64_t base = AHF_BLOCK; base < n && kept == n; base += 4 * AHF_BLOCK, buf ^= 1)
+    kept = group_cut_step<4>(K, base, n, l, cen, pv, s_first[buf]);
+  __syncthreads(); /* the words are the next halo's */
+  *od = sphere_ovdens(K, kept - 1, l[kept - 1], cen, pv, R);
+  *M = (double)kept;
+  return kept;
+}
+
+/*
+ * The haloes order[q0..nh) (order NULL: all, by index) into one list per form:
+ * list[f*nh ..), cnt[f] of them.  With the first rem_outsideRvir ahead of the
+ * unbinding its cut is made here, a workgroup a halo, and a halo goes to the
+ * form that holds what is left (a gathered halo keeps about one member in
+ * twenty): in the form of its full list the cut members would be carried
+ * through every iteration.  A halo that is chunked at any rate makes its cut
+ * there (pad: the cut is still to be made).  The record's fields are the
+ * cut's, or cleared.  (2.8 million gathered members, 2,400 haloes: 15 us; cut
+ * 1,024 members a step 50 us, for the records beyond the cut.)
+ */
+__global__ void __launch_bounds__(AHF_BLOCK) k_bin_forms(UnbindConst K, const int64_t *__restrict__ off,
+                                                  const int32_t *__restrict__ order, int64_t q0, int64_t nh,
+                                                  FormLeast least, const uint32_t *__restrict__ a,
+                                                  const double *__restrict__ cen, const float4 *__restrict__ pv,
+                                                  int32_t *__restrict__ list, int32_t *__restrict__ cnt,
+                                                  HaloOut *__restrict__ out)
+{
+  for (int64_t q = q0 + blockIdx.x; q < nh; q += gridDim.x) {
+    const int64_t h = order ? order[q] : q, o = off[h];
+    int64_t n = off[h + 1] - o;
+    HaloOut r;
+    memset(&r, 0, sizeof(r));
+    if (K.cut_before && n >= K.minpart) {
+      if (n < least.v[UF_CHUNK]) {
+        const double c3[3] = {cen[3 * h], cen[3 * h + 1], cen[3 * h + 2]};
+        n = group_cut(K, n, a + o, c3, pv, &r.M_vir, &r.R_vir, &r.ovdens);
+        r.set = AHFGPU_SET_MVIR | AHFGPU_SET_RVIR | AHFGPU_SET_PHI0 | AHFGPU_SET_OVDENS;
+      } else {
+        r.pad = 1;
+      }
+    }
+    if (threadIdx.x == 0) {
+      r.npart = n;
+      out[h] = r;
+      int f = 0;
+      while (f + 1 < UF_FORMS && n < least.v[f]) f++;
+      list[f * nh + atomicAdd(cnt + f, 1)] = (int32_t)h;
+    }
+  }
 }
 
 /* plain form: one halo per launch */
-template <int BS>
-__global__ void __launch_bounds__(BS) k_unbind_one(UnbindConst K, int64_t h, const int64_t *__restrict__ off,
-                                                   const int64_t *__restrict__ seed, uint32_t *a, uint32_t *b,
-                                                   double *dist, double *phi,
-                                                   uint8_t *st, Staged g, const double *__restrict__ cen,
-                                                   const float4 *__restrict__ pv,
-                                                   HaloOut *__restrict__ out)
+template <int BS, int IPT>
+__global__ void __launch_bounds__(BS, AHF_UNBIND_WAVES(IPT))
+    k_unbind_one(UnbindConst K, int64_t h, const int64_t *__restrict__ off, const int64_t *__restrict__ seed, uint32_t *a,
+                 uint32_t *b, double *dist, double *phi, uint8_t *st, Staged g, const double *__restrict__ cen,
+                 const float4 *__restrict__ pv, HaloOut *__restrict__ out)
 {
   const int64_t o = off[h], n = off[h + 1] - o;
   const double c3[3] = {cen[3 * h], cen[3 * h + 1], cen[3 * h + 2]};
   const Staged go = {g.dx + o, g.dy + o, g.dz + o, g.vx + o, g.vy + o, g.vz + o};
-  unbind_halo<BS, AHF_UNBIND_IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
+  unbind_form<BS, IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
 }
 
 __global__ void k_sorted_out(const int64_t *__restrict__ off, int64_t nh, HaloOut *__restrict__ out)
@@ -1049,7 +1814,15 @@ __global__ void k_copy_u32(const uint32_t *__restrict__ in, int64_t n, uint32_t 
  * kernel's; the certified bound of rec_eval holds for any order.
  */
 #define AHF_SPLIT_BLOCK 512
-#define AHF_SPLIT_DEFAULT 16384 /* default split_min */
+/* the default split_min: once one halo is this large, every halo that the
+ * register forms do not hold goes to the split path; else the chunked form
+ * takes them.  The path costs some 0.5 ms whatever it is given (the graph, the
+ * launches of five or six iterations); the chunked form 15 us for each 2048
+ * members and iteration of its largest halo.  2,000 isolated haloes (largest
+ * 171,870): 0.70 ms with all from 4097 members on split, 0.86 with those from
+ * 16384; a 256^3 box's gathered haloes (largest 8,000): 0.48 ms chunked, 0.61
+ * split. */
+#define AHF_SPLIT_FIRST 16384
 #define AHF_TILE 1024 /* members per tile: 256 threads x 4 */
 
 struct SplitHalo {
@@ -1233,7 +2006,7 @@ __global__ void __launch_bounds__(256) k_sp_spec_tot(const SplitHalo *__restrict
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int64_t e = H.o + j0 + i;
-    if (j0 + i < H.n && st[e]) {
+    if (j0 + i < H.n && (st[e] & 1)) {
       run.x += (double)g.vx[e]; run.y += (double)g.vy[e]; run.z += (double)g.vz[e]; run.m += 1.0;
     }
   }
@@ -1291,17 +2064,19 @@ __global__ void __launch_bounds__(256) k_sp_spec_eval(UnbindConst K, const Split
   const int64_t j0 = T.j0 + (int64_t)threadIdx.x * 4;
   int bj[4], b0[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) bj[i] = b0[i] = j0 + i < n ? (int)st[o + j0 + i] : 0;
+  for (int i = 0; i < 4; i++) bj[i] = b0[i] = j0 + i < n ? (int)(st[o + j0 + i] & 1) : 0;
   D4 tot;
   int unc = 0, sweeps = 0, ev = 0;
-  settle_chunk<256, 4>(K, n, T.j0, dist + o, phi + o, go, Phi0, tcv[blockIdx.x], B, bj, &tot, &unc, &sweeps, sh4,
+  uint32_t ub = 0;
+  settle_chunk<256, 4>(K, n, T.j0, dist + o, phi + o, go, Phi0, tcv[blockIdx.x], B, bj, &tot, &unc, &ub, &sweeps, sh4,
                        sflag, ev);
   int chg = 0;
 #pragma unroll
   for (int i = 0; i < 4; i++)
     if (j0 + i < n) {
       chg |= bj[i] != b0[i];
-      st[o + j0 + i] = (uint8_t)bj[i];
+      /* bit 1: an uncertain test, for exact_iteration (cleared there) */
+      st[o + j0 + i] = (uint8_t)(bj[i] | ((ub >> i) & 1u) << 1);
     }
   if (chg) atomicOr(&s_chg, 1);
   __syncthreads();
@@ -1365,7 +2140,7 @@ __global__ void __launch_bounds__(256) k_sp_spec_resume(SplitHalo *sh, const int
 /* the recurrence of one iteration, one workgroup per active split halo;
  * with spec, from where the speculative passes leave it */
 __global__ void __launch_bounds__(AHF_SPLIT_BLOCK) k_sp_rec(UnbindConst K, SplitHalo *sh, const double *dist,
-                                                            const double *phi, uint8_t *st, Staged g, int spec)
+                                                            double *phi, uint8_t *st, Staged g, int spec)
 {
   SplitHalo &H = sh[blockIdx.x];
   if (!H.active) return;
@@ -2317,7 +3092,7 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
   uint8_t *st = A.get<uint8_t>(ne);
   Staged g = {A.get<double>(ne), A.get<double>(ne), A.get<double>(ne),
               A.get<float>(ne), A.get<float>(ne), A.get<float>(ne)};
-  int32_t *next = A.get<int32_t>(3);
+  int32_t *next = A.get<int32_t>(2 * UF_FORMS); /* the forms' queue counters, their lists' lengths */
   int64_t *seed = A.get<int64_t>(nh);
   if (!k0 || !k1 || !v0 || !v1 || !hk0 || !hk1 || !rtmp || !s->buf_a || !s->buf_b || !dist || !phi || !st ||
       !s->out || !next || !seed || !g.dx || !g.dy || !g.dz || !g.vx || !g.vy || !g.vz)
@@ -2445,49 +3220,89 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     /* nothing more */
   } else if (run == 0) {
     /* the order is largest first: haloes of split_min members or more take
-     * the split path on the second stream; of the rest, haloes of
-     * AHF_BIG_HALO members or more get AHF_BIG_BLOCK-thread workgroups, the
-     * others AHF_BLOCK */
-    int64_t nbig = 0, nsplit = 0;
+     * the split path on the second stream, the others the forms by size: the
+     * wavefront forms on the third stream, the workgroup forms on the first,
+     * the chunked one (only with split_min above its size) behind the split
+     * path's start */
+    int64_t nsplit = 0;
     const std::vector<int32_t> &ord = s->h_ord;
-    const int64_t split_min = c->split_min > 0 ? c->split_min : AHF_SPLIT_DEFAULT;
+    const int64_t largest = nh ? s->h_off[ord[0] + 1] - s->h_off[ord[0]] : 0;
+    const int64_t split_min = c->split_min > 0 ? c->split_min : largest >= AHF_SPLIT_FIRST ? AHF_BIG_MOST + 1 : INT64_MAX;
     auto size_of = [&](int64_t q) { return s->h_off[ord[q] + 1] - s->h_off[ord[q]]; };
     if (c->split_min >= 0)
       while (nsplit < nh && size_of(nsplit) >= split_min && size_of(nsplit) >= p->minpart) nsplit++;
-    const int64_t big_halo = c->big_halo > 0 ? c->big_halo : AHF_BIG_HALO;
-    const int64_t wave_halo = c->wave_halo > 0 ? std::min<int64_t>(c->wave_halo, big_halo) : AHF_WAVE_HALO;
-    while (nbig < nh && size_of(nbig) >= big_halo) nbig++;
-    if (nbig < nsplit) nbig = nsplit;
-    /* haloes below AHF_WAVE_HALO members: one wavefront each */
-    int64_t nmid = nbig;
-    while (nmid < nh && size_of(nmid) >= wave_halo) nmid++;
-    hipMemsetAsync(next, 0, 3 * sizeof(int32_t), c->st);
-    /* the second and third streams start after the sort, the seeds and the
-     * queue counters */
-    hipEventRecord(c->ev_s0, c->st);
-    if (nbig > nsplit) {
-      const int64_t grid = std::min<int64_t>(nbig - nsplit, (int64_t)dev_cu * 2);
-      hipLaunchKernelGGL(k_unbind_batched<AHF_BIG_BLOCK>, dim3((unsigned)grid), dim3(AHF_BIG_BLOCK), 0, c->st, K,
-                         s->off, s->order, nsplit, nbig, next, seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);
+    int64_t q0[UF_FORMS + 1] = {nsplit};
+    for (int f = 0; f < UF_FORMS; f++) {
+      const int64_t least = uf_least(c, f);
+      q0[f + 1] = std::lower_bound(ord.begin() + q0[f], ord.end(), least, [&](int32_t h, int64_t v) {
+                    return s->h_off[h + 1] - s->h_off[h] >= v;
+                  }) - ord.begin();
     }
-    if (nmid > nbig) {
-      const int64_t grid = std::min<int64_t>(nmid - nbig, (int64_t)dev_cu * 8);
-      hipLaunchKernelGGL(k_unbind_batched<AHF_BLOCK>, dim3((unsigned)grid), dim3(AHF_BLOCK), 0, c->st, K, s->off,
-                         s->order, nbig, nmid, next + 1, seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);
+    hipMemsetAsync(next, 0, 2 * UF_FORMS * sizeof(int32_t), c->st);
+    /* with the cut ahead of the unbinding the forms' lists are made on the
+     * device, from what the cut leaves: a form may then hold any halo of its
+     * size or more */
+    const bool binned = K.cut_before != 0 && nh > nsplit;
+    UnbindConst KF = K;
+    FormLeast least;
+    for (int f = 0; f < UF_FORMS; f++) least.v[f] = uf_least(c, f);
+    int32_t *list = nullptr, *cnt = next + UF_FORMS;
+    const bool either = uf_either(binned, binned ? nh - nsplit : q0[UF_FORMS] - q0[UF_WAVE], dev_cu);
+    if (either) least.v[UF_WAVE] = 0;
+    /* the split path is used where one halo needs it (below); its haloes take
+     * the cut there */
+    auto most = [&](int f) { return binned ? q0[f + 1] - nsplit : q0[f + 1] - q0[f]; };
+    if (binned) {
+      list = A.get<int32_t>(UF_FORMS * nh);
+      if (!list) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (unbinding)");
+      hipLaunchKernelGGL(k_bin_forms, dim3((unsigned)std::min<int64_t>(nh - nsplit, (int64_t)dev_cu * 8)), dim3(AHF_BLOCK), 0, c->st,
+                         K, s->off, s->order, nsplit, nh, least, s->buf_a, s->cen, c->pv, list, cnt, s->out);
+      KF.cut_before = CUT_DONE;
     }
-    if (nh > nmid && nmid == 0) {
-      /* only one-wavefront haloes: on the first stream, no hand-over */
-      const int64_t grid = std::min<int64_t>(nh, (int64_t)dev_cu * 32);
-      hipLaunchKernelGGL(k_unbind_batched<64>, dim3((unsigned)grid), dim3(64), 0, c->st, K, s->off, s->order, 0, nh,
-                         next + 2, seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);
-    } else if (nh > nmid) {
-      const int64_t grid = std::min<int64_t>(nh - nmid, (int64_t)dev_cu * 32);
-      hipStreamWaitEvent(c->st3, c->ev_s0, 0);
-      hipLaunchKernelGGL(k_unbind_batched<64>, dim3((unsigned)grid), dim3(64), 0, c->st3, K, s->off, s->order, nmid,
-                         nh, next + 2, seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);
-      hipEventRecord(c->ev_s2, c->st3);
-      hipStreamWaitEvent(c->st, c->ev_s2, 0);
+    /* the other streams start after the sort, the seeds and the queue
+     * counters; with a single form and no split path there is no hand-over */
+    const int64_t wgs = q0[UF_WAVE] - nsplit, wvs = binned ? nh - nsplit : q0[UF_FORMS] - q0[UF_WAVE];
+    const bool fork = nsplit > 0 || (wgs > 0 && wvs > 0) || (q0[UF_BIG] > nsplit && nh > q0[UF_BIG]);
+    if (fork) hipEventRecord(c->ev_s0, c->st);
+    /* F: the form's counters; Q: its first halo in the host's order */
+#define AHF_UNBIND_LAUNCH(F, Q, N, BS, IPT, PER_CU, STREAM)                                                              \
+  do {                                                                                                                   \
+    const dim3 grid_((unsigned)std::min<int64_t>((N), (int64_t)dev_cu * (PER_CU)));                                      \
+    if (binned)                                                                                                          \
+      hipLaunchKernelGGL((k_unbind_dq<BS, IPT>), grid_, dim3(BS), 0, STREAM, KF, s->off, list + (F) * nh, cnt + (F),      \
+                         next + (F), seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);                 \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((k_unbind<BS, IPT>), grid_, dim3(BS), 0, STREAM, KF, s->off, s->order, q0[F], (Q), next + (F),   \
+                         seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);                             \
+  } while (0)
+    hipStream_t sw = fork ? c->st3 : c->st;
+    if (most(UF_CHUNK) > 0) {
+      if (fork) hipStreamWaitEvent(c->st2, c->ev_s0, 0);
+      AHF_UNBIND_LAUNCH(UF_CHUNK, q0[UF_BIG], most(UF_CHUNK), AHF_BIG_BLOCK, 0, 2, fork ? c->st2 : c->st);
+      if (fork) hipEventRecord(c->ev_s1, c->st2);
     }
+    /* binned, every form may hold long-running haloes: the middle one on
+     * another stream than the big one's, the second if nothing else is there */
+    const bool mid2 = binned && fork && nsplit == 0 && most(UF_CHUNK) == 0 && most(UF_BIG) > 0;
+    hipStream_t sm = mid2 ? c->st2 : binned && fork && wvs > 0 && most(UF_BIG) > 0 ? sw : c->st;
+    if (wvs > 0 && fork) hipStreamWaitEvent(sw, c->ev_s0, 0);
+    if (mid2) hipStreamWaitEvent(c->st2, c->ev_s0, 0);
+    if (sm == c->st && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, c->st);
+    if (most(UF_MID) > 0) AHF_UNBIND_LAUNCH(UF_MID, q0[UF_WAVE], most(UF_MID), AHF_BLOCK, 8, 2, sm);
+    if (mid2) hipEventRecord(c->ev_s1, c->st2);
+    if (wvs > 0) {
+      if (either) {
+        AHF_UNBIND_LAUNCH(UF_WAVE, nh, wvs, 64, UF_EITHER, 8, sw);
+      } else {
+        if (most(UF_WAVE) > 0) AHF_UNBIND_LAUNCH(UF_WAVE, q0[UF_SMALL], most(UF_WAVE), 64, 8, 8, sw);
+        if (most(UF_SMALL) > 0) AHF_UNBIND_LAUNCH(UF_SMALL, nh, most(UF_SMALL), 64, 2, 16, sw);
+      }
+      if (fork) hipEventRecord(c->ev_s2, sw);
+    }
+    if (sm != c->st && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, c->st);
+    if (fork && (mid2 || most(UF_CHUNK) > 0)) hipStreamWaitEvent(c->st, c->ev_s1, 0);
+    if (fork && wvs > 0) hipStreamWaitEvent(c->st, c->ev_s2, 0);
+#undef AHF_UNBIND_LAUNCH
     if (nsplit > 0) {
       int rc = split_unbind(c, K, s, ord.data(), nsplit, seed, dist, phi, st, g);
       if (rc) return rc;
@@ -2496,13 +3311,14 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     /* plain form: one halo per launch, results synchronised per halo as a
      * per-call rem_unbound() would need them */
     for (int64_t h = 0; h < nh; h++) {
-      if (s->h_off[h + 1] - s->h_off[h] >= (c->big_halo > 0 ? c->big_halo : AHF_BIG_HALO))
-        hipLaunchKernelGGL(k_unbind_one<AHF_BIG_BLOCK>, dim3(1), dim3(AHF_BIG_BLOCK), 0, c->st, K, h, s->off,
-                           seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv,
-                           s->out);
-      else
-        hipLaunchKernelGGL(k_unbind_one<AHF_BLOCK>, dim3(1), dim3(AHF_BLOCK), 0, c->st, K, h, s->off, seed,
-                           s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);
+      const int64_t n = s->h_off[h + 1] - s->h_off[h];
+#define AHF_UNBIND_ONE(BS, IPT)                                                                                   \
+  hipLaunchKernelGGL((k_unbind_one<BS, IPT>), dim3(1), dim3(BS), 0, c->st, K, h, s->off, seed, s->buf_a, s->buf_b, \
+                     dist, phi, st, g, s->cen, c->pv, s->out)
+      if (n > AHF_BIG_MOST) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 0);
+      else if (n >= uf_least(c, UF_BIG)) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 8);
+      else AHF_UNBIND_ONE(AHF_BLOCK, 8);
+#undef AHF_UNBIND_ONE
       hipStreamSynchronize(c->st);
     }
   }
@@ -2626,10 +3442,9 @@ extern "C" void ahfgpu_release_halos(ahfgpu_ctx *c)
  * when a context is created there (ahf_noalloc_init).  Nothing here calls
  * hipMalloc or hipFree.  The steps are those of ahfgpu_unbind in the
  * batched mode with every halo in the persistent kernel, all laid out on
- * the device: the largest-first queue order (a stable radix sort of the
- * sizes), its tier bounds, the radial sort (stable radix sorts on the
- * distance key and then the halo), the seeds, the three persistent tiers,
- * and the copy of the results into the caller's arrays.
+ * the device: the radial sort (stable radix sorts on the distance key and
+ * then the halo), the seeds, the lists of the unbinding's forms by size, the
+ * persistent forms, and the copy of the results into the caller's arrays.
  */
 #define AHF_NA_SCRATCH_BYTES ((size_t)192 << 20)
 #define AHF_NA_MAX_DEVICES 64
@@ -2642,7 +3457,7 @@ static std::mutex g_na_mu;
 /* byte offsets of the arrays of one call inside scratch */
 struct NaLayout {
   size_t k0, k1, v0, v1, hk0, hk1, rtmp, a, b, dist, phi, st, dx, dy, dz, vx, vy, vz;
-  size_t ok0, ok1, ov0, ov1, ortmp, seed, out, qb, words;
+  size_t list, seed, out, words;
   size_t tie, tpos, tmp32h, tiew, tiew_bytes; /* the indexx replay of haloes with equal distances */
   size_t total;
 };
@@ -2675,15 +3490,10 @@ static NaLayout na_layout(int64_t nh, int64_t ne)
   L.vx = take(m * 4);
   L.vy = take(m * 4);
   L.vz = take(m * 4);
-  L.ok0 = take(h * 4);
-  L.ok1 = take(h * 4);
-  L.ov0 = take(h * 4);
-  L.ov1 = take(h * 4);
-  L.ortmp = take((size_t)radix_tmp_u32<uint32_t>((int64_t)h) * 4);
+  L.list = take(UF_FORMS * h * 4);
   L.seed = take(h * 8);
   L.out = take(h * sizeof(HaloOut));
-  L.qb = take(4 * sizeof(int64_t));
-  L.words = take(8 * sizeof(int32_t));
+  L.words = take((1 + 2 * UF_FORMS) * sizeof(int32_t));
   L.tie = take(h);
   L.tpos = take((h + 1) * 4);
   L.tmp32h = take((size_t)scan_tmp_elems((int64_t)h) * 4 + 64);
@@ -2736,45 +3546,6 @@ __global__ void k_na_check(const int64_t *__restrict__ off, int64_t nh, int64_t 
     if (!ok) atomicOr(bad, 1);
   }
   if (i < ne && (int64_t)ip[i] >= N) atomicOr(bad, 2);
-}
-
-/* queue order: sizes as descending keys, a stable sort keeps equal sizes in
- * index order (as the host's stable sort does) */
-__global__ void k_na_order_keys(const int64_t *__restrict__ off, int64_t nh, uint32_t *__restrict__ key,
-                                uint32_t *__restrict__ val)
-{
-  const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= nh) return;
-  key[h] = 0xFFFFFFFFu - (uint32_t)(off[h + 1] - off[h]);
-  val[h] = (uint32_t)h;
-}
-
-/* the first queue position whose halo has fewer than `lim` members (sizes do
- * not increase along the queue) */
-__device__ inline int64_t na_first_below(const int64_t *off, const int32_t *order, int64_t nh, int64_t lim)
-{
-  int64_t lo = 0, hi = nh;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    const int32_t h = order[mid];
-    if (off[h + 1] - off[h] >= lim) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-/* tier bounds of the persistent kernels and their queue counters */
-__global__ void k_na_bounds(const int64_t *__restrict__ off, const int32_t *__restrict__ order, int64_t nh,
-                            int64_t big_halo, int64_t wave_halo, int64_t *__restrict__ qb, int32_t *__restrict__ next)
-{
-  if (threadIdx.x != 0) return;
-  const int64_t nbig = na_first_below(off, order, nh, big_halo);
-  int64_t nmid = na_first_below(off, order, nh, wave_halo);
-  if (nmid < nbig) nmid = nbig;
-  qb[0] = 0;
-  qb[1] = nbig;
-  qb[2] = nmid;
-  qb[3] = nh;
-  next[0] = next[1] = next[2] = 0;
 }
 
 /* radial sort keys of all members: dist^2 where the halo is sorted, 0 where
@@ -2870,33 +3641,23 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
   uint8_t *stt = (uint8_t *)(base + L.st);
   const Staged g = {(double *)(base + L.dx), (double *)(base + L.dy), (double *)(base + L.dz),
                     (float *)(base + L.vx),  (float *)(base + L.vy),  (float *)(base + L.vz)};
-  uint32_t *ok0 = (uint32_t *)(base + L.ok0), *ok1 = (uint32_t *)(base + L.ok1);
-  uint32_t *ov0 = (uint32_t *)(base + L.ov0), *ov1 = (uint32_t *)(base + L.ov1);
-  uint32_t *ortmp = (uint32_t *)(base + L.ortmp);
+  int32_t *list = (int32_t *)(base + L.list);
   int64_t *seed = (int64_t *)(base + L.seed);
   HaloOut *hout = (HaloOut *)(base + L.out);
-  int64_t *qb = (int64_t *)(base + L.qb);
-  int32_t *words = (int32_t *)(base + L.words); /* [0..2] queue counters, [3] input check */
+  int32_t *words = (int32_t *)(base + L.words); /* [0] input check, then the forms' queue counters and their lists' lengths */
   /* the caller's offsets and members are checked before anything reads
    * through them; scratch keeps the last call's contents, so the check
    * word is cleared first */
-  hipLaunchKernelGGL(k_na_zero, dim3(1), dim3(64), 0, st, words, 8);
+  hipLaunchKernelGGL(k_na_zero, dim3(1), dim3(64), 0, st, words, 1 + 2 * UF_FORMS);
   const int64_t nchk = std::max<int64_t>(nh + 1, ne);
-  hipLaunchKernelGGL(k_na_check, dim3(nb_of(nchk)), dim3(AHF_BLOCK), 0, st, off, nh, ne, members, c->N, words + 3);
+  hipLaunchKernelGGL(k_na_check, dim3(nb_of(nchk)), dim3(AHF_BLOCK), 0, st, off, nh, ne, members, c->N, words);
   int32_t bad = 0;
-  if (hipMemcpyAsync(&bad, words + 3, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
+  if (hipMemcpyAsync(&bad, words, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return c->fail(AHFGPU_EHIP, "ahfgpu_unbind_noalloc: input check: %s", hipGetErrorString(hipGetLastError()));
   if (bad & 1) return c->fail(AHFGPU_EINVAL, "ahfgpu_unbind_noalloc: offsets must start at 0 and not decrease");
   if (bad & 2) return c->fail(AHFGPU_EINVAL, "ahfgpu_unbind_noalloc: a member refers to a particle beyond the resident set");
   const UnbindConst K = unbind_const(p, mode, band);
-  /* largest first, and the tier bounds */
-  hipLaunchKernelGGL(k_na_order_keys, dim3(nb_of(nh)), dim3(AHF_BLOCK), 0, st, off, nh, ok0, ov0);
-  const int wo = radix_sort<uint32_t, uint32_t>(ok0, ov0, ok1, ov1, nh, 32, ortmp, st);
-  const int32_t *order = (const int32_t *)(wo ? ov1 : ov0);
-  const int64_t big_halo = c->big_halo > 0 ? c->big_halo : AHF_BIG_HALO;
-  const int64_t wave_halo = c->wave_halo > 0 ? std::min<int64_t>(c->wave_halo, big_halo) : AHF_WAVE_HALO;
-  hipLaunchKernelGGL(k_na_bounds, dim3(1), dim3(64), 0, st, off, order, nh, big_halo, wave_halo, qb, words);
   /* radial sort (or the lists as given) into buf_a */
   const bool sort_only = (mode & AHFGPU_UNBIND_SORT_ONLY) != 0;
   const bool no_sort = (mode & (AHFGPU_UNBIND_NO_SORT | AHFGPU_UNBIND_RVIR_ONLY)) != 0;
@@ -2937,18 +3698,37 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
                          seed);
     int dev_cu = 256;
     hipDeviceGetAttribute(&dev_cu, hipDeviceAttributeMultiprocessorCount, c->device);
-    /* the one-wavefront tier on the third stream, as in the batched form */
+    /* the forms on the three streams, as in the batched form, over lists made
+     * on the device (with the cut ahead of the unbinding, if any) */
+    FormLeast least;
+    for (int f = 0; f < UF_FORMS; f++) least.v[f] = uf_least(c, f);
+    const bool either = uf_either(true, nh, dev_cu);
+    if (either) least.v[UF_WAVE] = 0;
+    int32_t *next = words + 1, *cnt = next + UF_FORMS;
+    hipLaunchKernelGGL(k_bin_forms, dim3((unsigned)std::min<int64_t>(nh, (int64_t)dev_cu * 8)), dim3(AHF_BLOCK), 0, st, K, off,
+                       (const int32_t *)nullptr, (int64_t)0, nh, least, buf_a, centres, c->pv, list, cnt, hout);
+    UnbindConst KF = K;
+    if (K.cut_before) KF.cut_before = CUT_DONE;
     hipEventRecord(c->ev_s0, st);
+    hipStreamWaitEvent(c->st2, c->ev_s0, 0);
     hipStreamWaitEvent(c->st3, c->ev_s0, 0);
-    hipLaunchKernelGGL(k_unbind_batched_dq<AHF_BIG_BLOCK>, dim3((unsigned)std::min<int64_t>(nh, 2 * dev_cu)),
-                       dim3(AHF_BIG_BLOCK), 0, st, K, off, order, qb, 0, words, seed, buf_a, buf_b, dist, phi, stt, g,
-                       centres, c->pv, hout);
-    hipLaunchKernelGGL(k_unbind_batched_dq<AHF_BLOCK>, dim3((unsigned)std::min<int64_t>(nh, 8 * dev_cu)),
-                       dim3(AHF_BLOCK), 0, st, K, off, order, qb, 1, words + 1, seed, buf_a, buf_b, dist, phi, stt, g,
-                       centres, c->pv, hout);
-    hipLaunchKernelGGL(k_unbind_batched_dq<64>, dim3((unsigned)std::min<int64_t>(nh, 32 * dev_cu)), dim3(64), 0,
-                       c->st3, K, off, order, qb, 2, words + 2, seed, buf_a, buf_b, dist, phi, stt, g, centres, c->pv, hout);
+#define AHF_UNBIND_LAUNCH(F, BS, IPT, PER_CU, STREAM)                                                             \
+  hipLaunchKernelGGL((k_unbind_dq<BS, IPT>), dim3((unsigned)std::min<int64_t>(nh, (int64_t)dev_cu * (PER_CU))),   \
+                     dim3(BS), 0, STREAM, KF, off, list + (F) * nh, cnt + (F), next + (F), seed, buf_a, buf_b,    \
+                     dist, phi, stt, g, centres, c->pv, hout);
+    AHF_UNBIND_LAUNCH(UF_CHUNK, AHF_BIG_BLOCK, 0, 2, c->st2)
+    if (either) {
+      AHF_UNBIND_LAUNCH(UF_WAVE, 64, UF_EITHER, 8, c->st3)
+    } else {
+      AHF_UNBIND_LAUNCH(UF_WAVE, 64, 8, 8, c->st3)
+      AHF_UNBIND_LAUNCH(UF_SMALL, 64, 2, 16, c->st3)
+    }
+    AHF_UNBIND_LAUNCH(UF_BIG, AHF_BIG_BLOCK, 8, 1, st)
+    AHF_UNBIND_LAUNCH(UF_MID, AHF_BLOCK, 8, 2, st)
+#undef AHF_UNBIND_LAUNCH
+    hipEventRecord(c->ev_s1, c->st2);
     hipEventRecord(c->ev_s2, c->st3);
+    hipStreamWaitEvent(st, c->ev_s1, 0);
     hipStreamWaitEvent(st, c->ev_s2, 0);
   }
   hipLaunchKernelGGL(k_na_out_halo, dim3(nb_of(nh)), dim3(AHF_BLOCK), 0, st, hout, nh, npart_out, props_out);

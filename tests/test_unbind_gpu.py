@@ -229,6 +229,143 @@ def test_schedule_variants(oracle, snapgen, ctx, tmp_path, sched):
         ctx.set_schedule(**before)
 
 
+FORM_SIZES = [19, 20, 21, 63, 64, 65, 127, 128, 129, 255, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8193,
+              16383, 16385]
+
+
+def _form_snapshot(path, seed):
+    """one isolated halo of each size around the forms' bounds: radii of a
+    cuspy profile, velocities with a tail above the escape speed, one halo
+    across the periodic corner, one with members on its centre, one that
+    loses every member"""
+    rng = np.random.default_rng(seed)
+    pos, mom, lists, cen, n0 = [], [], [], [], 0
+    for i, n in enumerate(FORM_SIZES):
+        c = np.array([0.0, 0.9999, 0.0001]) if i == 5 else rng.uniform(0.05, 0.95, 3)
+        r = 0.01 * rng.random(n) ** 1.5
+        d = rng.normal(size=(n, 3))
+        p = c + r[:, None] * d / np.linalg.norm(d, axis=1)[:, None]
+        if i == 8:
+            p[:3] = np.float32(c).astype(np.float64)
+            c = np.float32(c).astype(np.float64)
+        v = rng.normal(0.0, 1.0, (n, 3)) * np.sqrt(n) * 2e-3 + rng.normal(0.0, 3.0, 3)
+        v[rng.random(n) < 0.15] *= 3.0
+        if i == 12:
+            v *= 1e4
+        pos.append(p % 1.0)
+        mom.append(v)
+        lists.append((rng.permutation(n) + n0).astype(np.uint64))
+        cen.append(c)
+        n0 += n
+    pos = np.concatenate(pos).astype(np.float32)
+    pos[pos >= 1.0] = 0.0
+    dumps.write_snapshot(path, pos, np.concatenate(mom), boxsize=1.0, pmass=1e8, L_dom=16, centres=np.array(cen),
+                         halo_lists=lists, r_fac=1.0, v_fac=1.0, phi_fac=2e-7, hubble=10.0, ovlim=200.0, rho_vir=6e13,
+                         gather_rad=np.full(len(lists), 0.02))
+
+
+@pytest.mark.parametrize("cuts", [0, WITH_RVIR])
+@pytest.mark.parametrize("plain,split,band,sched", [(0, 0, 0.0, {}), (0, -1, 0.0, {}), (1, 0, 0.0, {}), (0, -1, 3e-2, {}),
+                                                    (0, -1, 0.0, dict(big_halo=600, wave_halo=70)), (0, 300, 0.0, {})])
+def test_form_sizes(oracle, ctx, tmp_path, cuts, plain, split, band, sched):
+    """haloes on both sides of every size at which the unbinding changes its
+    form, in every form that can hold them, some sent to the exact replay"""
+    snap, out = str(tmp_path / "f.snap"), str(tmp_path / "o.halo")
+    _form_snapshot(snap, 5)
+    dump = oracle.oracle_construct_dump if cuts else oracle.oracle_unbind_dump
+    assert dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    lost = np.array(FORM_SIZES) - ref.npart.astype(int)
+    assert lost[12] >= FORM_SIZES[12] - 1 and np.sum(lost > 0) > len(FORM_SIZES) // 2
+    s = dumps.read_snapshot(snap)
+    before = ctx.schedule()
+    try:
+        ctx.set_schedule(**sched)
+        ctx.set_unbind_split(split)
+        ctx.set_particles(s.pos, s.mom)
+        ctx.set_halos(s.centre, s.halo_npart, s.ipart)
+        info = ctx.unbind(s.minpart, s.vtune, s.r_fac, s.v_fac, s.phi_fac, s.hubble, mode=plain | cuts, band=band,
+                          ovlim=s.ovlim, rho_vir=s.rho_vir, rho_fac=s.rho_fac)
+        npart, props, lists = ctx.unbind_results()
+    finally:
+        ctx.set_schedule(**before)
+        ctx.set_unbind_split(0)
+    assert band == 0.0 or info.n_exact_replays > 5
+    _compare(ref, npart, props, lists, f"forms {cuts} {plain} {split} {band} {sched}")
+    if cuts:
+        assert np.array_equal(ref.ovdens, props[:, 3])
+
+
+def _edge_halo(rng, n, phi_fac, vtune2, minpart):
+    """positions (offsets) and velocities of a halo in radial order, one of
+    whose members sits within about one unit of rounding of the bound test as
+    rem_unbound's sequential sums evaluate it: vx and vy from candidates just
+    below the limit, vz (no other member has one) makes up the rest"""
+    r = np.sort(rng.uniform(1e-4, 1e-2, n))
+    d = rng.normal(size=(n, 3))
+    off = np.round(r[:, None] * d / np.linalg.norm(d, axis=1)[:, None] * 2.0 ** 24) / 2.0 ** 24
+    dist = np.sqrt(off[:, 0] * off[:, 0] + off[:, 1] * off[:, 1] + off[:, 2] * off[:, 2])
+    o = np.argsort(dist)
+    off, dist = off[o], dist[o]
+    phi, acc, ip, dp = [], 0.0, 0.0, 0.0
+    for j, x in enumerate(dist.tolist()):
+        cur = float(j + 1) / (x * x)
+        acc += (cur + ip) / 2. * (x - dp)
+        phi.append(acc)
+        ip, dp = cur, x
+    phi0 = acc + float(n) / dist[-1]
+    lim = vtune2 * (2 * np.abs(np.array(phi) - phi0) * phi_fac)
+    v = np.zeros((n, 3), np.float32)
+    v[:, :2] = rng.normal(0.0, 0.3, (n, 2)) * np.sqrt(lim)[:, None] + rng.normal(0.0, 0.2, 2) * np.sqrt(lim[-1])
+    v2 = v[:minpart // 2, 0] * v[:minpart // 2, 0] + v[:minpart // 2, 1] * v[:minpart // 2, 1]
+    js = int(np.argsort(v2)[minpart // 2 // 2 - 1])
+    V, M = [float(v[js, 0]), float(v[js, 1])], 1.0
+    for j in range(n):
+        if j == n // 2:
+            ang, k = rng.uniform(0, 2 * np.pi, 4000), np.sqrt(lim[j])
+            cx, cy = np.float32(V[0] / M + k * np.cos(ang)), np.float32(V[1] / M + k * np.sin(ang))
+            dx, dy = cx.astype(np.float64) - V[0] / M, cy.astype(np.float64) - V[1] / M
+            rest = lim[j] - (dx * dx + dy * dy)
+            ok = (rest > 0) & (rest < 3e-8 * lim[j])
+            cx, cy, dx, dy, cz = cx[ok], cy[ok], dx[ok], dy[ok], np.float32(np.sqrt(rest[ok]))
+            gap = np.abs((dx * dx + dy * dy + cz.astype(np.float64) ** 2) - lim[j])
+            b = int(np.argmin(gap))
+            v[j] = cx[b], cy[b], cz[b]
+        x, y, z = (float(c) for c in v[j])
+        a, b, c = x - V[0] / M, y - V[1] / M, z
+        if not (a * a + b * b + c * c > lim[j]):
+            M += 1.0
+            V[0] += x
+            V[1] += y
+    return off, v
+
+
+@pytest.mark.parametrize("split", [0, -1, 300])
+def test_rounding_edge(oracle, ctx, tmp_path, split):
+    """members whose bound test AHF's own rounding decides: the parallel
+    sums' answer differs for some, the library's must not, in any form"""
+    rng = np.random.default_rng(11)
+    phi_fac, vtune, minpart = 1e-7, 1.5, 20
+    pos, mom, lists, cen, n0 = [], [], [], [], 0
+    for i, n in enumerate([60, 400, 1500, 3500, 7000, 12000] * 3):
+        off, v = _edge_halo(rng, n, phi_fac, vtune * vtune, minpart)
+        c = np.array([0.25 + 0.0625 * (i % 6), 0.5, 0.25 + 0.25 * (i // 6)])
+        pos.append(c + off)
+        mom.append(v)
+        lists.append((rng.permutation(n) + n0).astype(np.uint64))
+        cen.append(c)
+        n0 += n
+    snap, out = str(tmp_path / "e.snap"), str(tmp_path / "o.halo")
+    dumps.write_snapshot(snap, np.concatenate(pos), np.concatenate(mom), boxsize=1.0, pmass=1e8, L_dom=16,
+                         centres=np.array(cen), halo_lists=lists, r_fac=1.0, v_fac=1.0, phi_fac=phi_fac, hubble=0.0,
+                         vtune=vtune, minpart=minpart, gather_rad=np.full(len(lists), 0.02))
+    assert oracle.oracle_unbind_dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    info, (npart, props, lists) = _run_gpu(ctx, dumps.read_snapshot(snap), 0, split=split)
+    assert info.n_exact_replays >= 12
+    _compare(ref, npart, props, lists, f"edge split {split}")
+
+
 def test_schedule_file(tmp_path, monkeypatch):
     """a context applies the schedule file named by AHF_SCHEDULE"""
     import json
