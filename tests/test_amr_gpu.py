@@ -111,6 +111,24 @@ def test_marched_levels(oracle, ctx, tmp_path, L, per_node, clump):
     _check(oracle, ctx, snap, tmp_path, f"march{L}_{per_node}_{clump}", 0)
 
 
+@pytest.mark.parametrize("seed", [0, 5, 161])
+def test_final_lists(oracle, ctx, tmp_path, seed):
+    """the final lists with offsets or entries asked for alone; the last
+    level of seed 161 got its refinement's particles back"""
+    snap = str(tmp_path / "rb.snap")
+    fuzz_snapshot(snap, seed)
+    _check(oracle, ctx, snap, tmp_path, f"lists{seed}", 0)
+    info = _gpu_dump(ctx, snap, str(tmp_path / "again.grid"))
+    assert (info.rolled_back == 1) == (seed == 161)
+    for lev in range(info.n_levels):
+        both = ctx.amr_level(lev)
+        list0 = np.zeros_like(both["list0"])
+        lst = np.zeros(max(int(both["list0"][-1]), 1), np.uint32)
+        ctx._check(ctx.lib.ahfgpu_amr_level_copy(ctx.h, lev, None, None, None, list0.ctypes.data, None))
+        ctx._check(ctx.lib.ahfgpu_amr_level_copy(ctx.h, lev, None, None, None, None, lst.ctypes.data))
+        assert np.array_equal(list0, both["list0"]) and np.array_equal(lst[:int(list0[-1])], both["list"])
+
+
 @pytest.mark.parametrize("mode", [0, 2])
 @pytest.mark.parametrize("L,clump,dyadic", [(16, 2047, False), (16, 9000, False), (10, 20000, False), (16, 70000, False),
                                             (16, 20000, True), (10, 4000, True)])
