@@ -129,6 +129,20 @@ def test_final_lists(oracle, ctx, tmp_path, seed):
         assert np.array_equal(list0, both["list0"]) and np.array_equal(lst[:int(list0[-1])], both["list"])
 
 
+@pytest.mark.parametrize("n", [32, 33, 1024, 1025, 4096, 4097, 8193, 30000])
+def test_fine_buckets(oracle, ctx, tmp_path, n):
+    """a node's bucket at the edges of the three ways to split it among the
+    children (one thread, one wavefront, one workgroup in steps of 4096)"""
+    rng = np.random.default_rng(n)
+    lat = (np.stack(np.meshgrid(*[np.arange(16)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5) / 16
+    lat = lat[np.any(np.floor(lat * 16) != 7, axis=1)]
+    cell = (7 + 0.998 * rng.random((n, 3))) / 16
+    pos = np.concatenate([np.repeat(lat, 8, 0), cell]).astype(np.float32)
+    snap = str(tmp_path / "b.snap")
+    dumps.write_snapshot(snap, pos, L_dom=16, L_max=64, Nth_dom=4.0, Nth_ref=2.0)
+    _check(oracle, ctx, snap, tmp_path, f"bucket{n}", 0)
+
+
 @pytest.mark.parametrize("mode", [0, 2])
 @pytest.mark.parametrize("L,clump,dyadic", [(16, 2047, False), (16, 9000, False), (10, 20000, False), (16, 70000, False),
                                             (16, 20000, True), (10, 4000, True)])
