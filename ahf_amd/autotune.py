@@ -39,7 +39,7 @@ CANDIDATES = {
     "march_zn": [0, 8, 16],
     "big_halo": [0, 512, 1024],
     "wave_halo": [0, 128, 256],
-    "split_min": [0, 4097, 8192, 16384, 32768, 65536, -1],
+    "split_min": [0, 4097, 8192, 32768, 65536, -1],
     "graph_batch": [4, 2, 8],
     "split_spec": [3, 1, 2, 4, 6, -1],
     "prof_split": [2048, 512, 1024, 4096, 8192],

@@ -1080,6 +1080,7 @@ struct ResShared {
   int32_t cnt[NW], has[NW];
   int32_t flag[NW], moved[2][NW];
   unsigned long long first;
+  double seg[16], ex, loc; /* phi0_chunked */
 };
 
 __device__ __forceinline__ D4 add4(D4 a, D4 b) { return D4{a.x + b.x, a.y + b.y, a.z + b.z, a.m + b.m}; }
@@ -1235,8 +1236,61 @@ __device__ __forceinline__ void res_cut(const UnbindConst &K, uint32_t *alive, c
   __syncthreads();
 }
 
+/* waves of the workgroup that chunks a list of n members: the association of
+ * Phi0's sum goes by the list's size alone, whichever form holds it */
+__device__ __forceinline__ int phi0_waves(int64_t n) { return n >= 2048 ? 8 : n >= 512 ? 4 : 1; }
+
+/* Phi0 of n <= 4096 members from their mid-point terms, in unbind_halo's
+ * association (4 members a thread, scans over wavefronts, chunks of rw
+ * wavefronts one after the other).  With a close pair at the centre Phi0 is
+ * 10^4 times a potential difference, and v_esc^2 of the profiles shows its
+ * last bits. */
+template <int BS>
+__device__ __forceinline__ double phi0_chunked(int n, int rw, const double *term, double dlast, ResShared<BS / 64> &S)
+{
+  const int lane = threadIdx.x & 63, nseg = (n + 255) / 256;
+  for (int k = threadIdx.x >> 6; k < nseg; k += BS / 64) {
+    const int j0 = 256 * k + 4 * lane;
+    double loc[4], run = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      run += j0 + i < n ? term[j0 + i] : 0.0;
+      loc[i] = run;
+    }
+    double inc = run;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const double u = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += u;
+    }
+    double ex = __shfl_up(inc, 1, 64);
+    if (lane == 0) ex = 0.0;
+    if (lane == 63) S.seg[k] = inc;
+    if (k == nseg - 1) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (j0 + i == n - 1) {
+          S.ex = ex;
+          S.loc = loc[i];
+        }
+    }
+  }
+  __syncthreads();
+  double carry = 0.0, base = 0.0;
+  for (int k = 0; k < nseg - 1; k++) {
+    base += S.seg[k];
+    if ((k + 1) % rw == 0) {
+      carry += base;
+      base = 0.0;
+    }
+  }
+  const double r = ((carry + (base + S.ex)) + S.loc) + (double)n / dlast;
+  __syncthreads();
+  return r;
+}
+
 template <int BS, int IPT>
-__device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0, int64_t seed0, uint32_t *a, double *dist,
+__device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0, int rw, int64_t seed0, uint32_t *a, double *dist,
                                                 double *phi, uint8_t *st, Staged g, const double cen[3],
                                                 const float4 *__restrict__ pv, HaloOut *out)
 {
@@ -1300,7 +1354,17 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
     set = (set | AHFGPU_SET_MVIR | AHFGPU_SET_PHI0) & ~AHFGPU_SET_RVIR;
   }
   int nremove = unbind ? 4 : 0;
+  /* the members of the last iteration, for Phi0 */
+  uint32_t alive_i = 0;
+  int r0_i = 0, n_i = 0, exact_i = 0;
+  double dprev_i = 0.0, dlast_i = 0.0;
   while (nremove > 3) {
+    alive_i = alive;
+    r0_i = r0;
+    n_i = n;
+    dprev_i = dprev;
+    dlast_i = dlast;
+    exact_i = 0;
     niter++;
     pit += n;
     /* mid-point terms and their prefix sum Phi_j (kept in lm) */
@@ -1455,6 +1519,7 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
     if (res_or<BS>(ub != 0, S)) {
       /* the uncertain tests, over the members staged in list order */
       replays++;
+      exact_i = 1;
       int r = r0;
 #pragma unroll
       for (int i = 0; i < IPT; i++) {
@@ -1493,6 +1558,25 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
     }
     if ((double)n < (double)K.minpart) break;
   }
+  if (niter && !exact_i) {
+    int r = r0_i;
+    double dp = dprev_i;
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      if (!((alive_i >> i) & 1u)) continue;
+      double term = 0.0;
+      if (d[i] > MZERO) {
+        const double Ip = r > 0 && dp > MZERO ? (double)r / (dp * dp) : 0.0;
+        const double I_mid = ((double)(r + 1) / (d[i] * d[i]) + Ip) / 2.;
+        term = I_mid * (d[i] - dp);
+      }
+      phi[r] = term;
+      dp = d[i];
+      r++;
+    }
+    __syncthreads();
+    Phi0 = phi0_chunked<BS>(n_i, rw, phi, dlast_i, S);
+  }
   if (rvir_set) set |= AHFGPU_SET_RVIR;
   if (K.cut_after && n >= K.minpart) {
     res_cut<BS, IPT>(K, &alive, d, r0, n, &M_vir, &R_vir, &ovdens, S);
@@ -1530,14 +1614,14 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
  * memory */
 #define UF_EITHER 28
 template <int BS, int IPT>
-__device__ __forceinline__ void unbind_form(const UnbindConst &K, int64_t n, int64_t seed0, uint32_t *a, uint32_t *b,
+__device__ __forceinline__ void unbind_form(const UnbindConst &K, int64_t n, int rw, int64_t seed0, uint32_t *a, uint32_t *b,
                                             double *dist, double *phi, uint8_t *st, Staged g, const double cen[3],
                                             const float4 *__restrict__ pv, HaloOut *out)
 {
   if constexpr (IPT == UF_EITHER) {
-    if (n <= 2 * BS) unbind_resident<BS, 2>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
-    else unbind_resident<BS, 8>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
-  } else if constexpr (IPT > 0) unbind_resident<BS, IPT>(K, n, seed0, a, dist, phi, st, g, cen, pv, out);
+    if (n <= 2 * BS) unbind_resident<BS, 2>(K, n, rw, seed0, a, dist, phi, st, g, cen, pv, out);
+    else unbind_resident<BS, 8>(K, n, rw, seed0, a, dist, phi, st, g, cen, pv, out);
+  } else if constexpr (IPT > 0) unbind_resident<BS, IPT>(K, n, rw, seed0, a, dist, phi, st, g, cen, pv, out);
   else unbind_halo<BS, AHF_UNBIND_IPT>(K, n, seed0, a, b, dist, phi, st, g, cen, pv, out);
 }
 
@@ -1590,7 +1674,7 @@ static inline unsigned seed_blocks(int64_t nh)
  * kernels are bound by the serial chain of the longest halo's iterations, not
  * by memory: in registers an iteration has no pass over memory and one barrier
  * a hand-over.  Against chunks for every size (unbinding alone): 2,000 lists of
- * 20 to 100,000 members 0.78 -> 0.69 ms, 20,000 lists 1.9 -> 1.4 ms, and 16
+ * 20 to 100,000 members 0.82 -> 0.77 ms, 20,000 lists 1.74 -> 1.39 ms, and 16
  * lists end to end 213 -> 192 us.
  */
 enum { UF_CHUNK = 0, UF_BIG, UF_MID, UF_WAVE, UF_SMALL, UF_FORMS };
@@ -1645,7 +1729,7 @@ __device__ __forceinline__ void unbind_queue(const UnbindConst &K, const int64_t
     const int64_t o = off[h], n = K.cut_before == CUT_DONE ? out[h].npart : off[h + 1] - o;
     const double c3[3] = {cen[3 * h], cen[3 * h + 1], cen[3 * h + 2]};
     const Staged go = {g.dx + o, g.dy + o, g.dz + o, g.vx + o, g.vy + o, g.vz + o};
-    unbind_form<BS, IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
+    unbind_form<BS, IPT>(K, n, phi0_waves(off[h + 1] - o), seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
     __syncthreads();
   }
 }
@@ -1773,7 +1857,7 @@ __global__ void __launch_bounds__(BS, AHF_UNBIND_WAVES(IPT))
   const int64_t o = off[h], n = off[h + 1] - o;
   const double c3[3] = {cen[3 * h], cen[3 * h + 1], cen[3 * h + 2]};
   const Staged go = {g.dx + o, g.dy + o, g.dz + o, g.vx + o, g.vy + o, g.vz + o};
-  unbind_form<BS, IPT>(K, n, seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
+  unbind_form<BS, IPT>(K, n, phi0_waves(off[h + 1] - o), seed[h], a + o, b + o, dist + o, phi + o, st + o, go, c3, pv, out + h);
 }
 
 __global__ void k_sorted_out(const int64_t *__restrict__ off, int64_t nh, HaloOut *__restrict__ out)
@@ -1814,15 +1898,11 @@ __global__ void k_copy_u32(const uint32_t *__restrict__ in, int64_t n, uint32_t 
  * kernel's; the certified bound of rec_eval holds for any order.
  */
 #define AHF_SPLIT_BLOCK 512
-/* the default split_min: once one halo is this large, every halo that the
- * register forms do not hold goes to the split path; else the chunked form
- * takes them.  The path costs some 0.5 ms whatever it is given (the graph, the
- * launches of five or six iterations); the chunked form 15 us for each 2048
- * members and iteration of its largest halo.  2,000 isolated haloes (largest
- * 171,870): 0.70 ms with all from 4097 members on split, 0.86 with those from
- * 16384; a 256^3 box's gathered haloes (largest 8,000): 0.48 ms chunked, 0.61
- * split. */
-#define AHF_SPLIT_FIRST 16384
+/* the default split_min.  The path costs some 0.5 ms whatever it is given (the
+ * graph, the launches of five or six iterations); the chunked form 15 us for
+ * each 2048 members and iteration of its largest halo: a 256^3 box's gathered
+ * haloes (largest 8,000) take 0.48 ms chunked, 0.61 split. */
+#define AHF_SPLIT_DEFAULT 16384
 #define AHF_TILE 1024 /* members per tile: 256 threads x 4 */
 
 struct SplitHalo {
@@ -3226,8 +3306,7 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
      * path's start */
     int64_t nsplit = 0;
     const std::vector<int32_t> &ord = s->h_ord;
-    const int64_t largest = nh ? s->h_off[ord[0] + 1] - s->h_off[ord[0]] : 0;
-    const int64_t split_min = c->split_min > 0 ? c->split_min : largest >= AHF_SPLIT_FIRST ? AHF_BIG_MOST + 1 : INT64_MAX;
+    const int64_t split_min = c->split_min > 0 ? c->split_min : AHF_SPLIT_DEFAULT;
     auto size_of = [&](int64_t q) { return s->h_off[ord[q] + 1] - s->h_off[ord[q]]; };
     if (c->split_min >= 0)
       while (nsplit < nh && size_of(nsplit) >= split_min && size_of(nsplit) >= p->minpart) nsplit++;
@@ -3276,18 +3355,24 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
                          seed, s->buf_a, s->buf_b, dist, phi, st, g, s->cen, c->pv, s->out);                             \
   } while (0)
     hipStream_t sw = fork ? c->st3 : c->st;
-    if (most(UF_CHUNK) > 0) {
+    /* the chunked form has the second stream, or the first where the split
+     * path has that one; the big form is then beside the others on the third */
+    const bool chunk1 = most(UF_CHUNK) > 0 && nsplit > 0;
+    const bool chunk2 = most(UF_CHUNK) > 0 && !chunk1;
+    if (chunk2) {
       if (fork) hipStreamWaitEvent(c->st2, c->ev_s0, 0);
       AHF_UNBIND_LAUNCH(UF_CHUNK, q0[UF_BIG], most(UF_CHUNK), AHF_BIG_BLOCK, 0, 2, fork ? c->st2 : c->st);
       if (fork) hipEventRecord(c->ev_s1, c->st2);
     }
+    if (chunk1) AHF_UNBIND_LAUNCH(UF_CHUNK, q0[UF_BIG], most(UF_CHUNK), AHF_BIG_BLOCK, 0, 2, c->st);
     /* binned, every form may hold long-running haloes: the middle one on
      * another stream than the big one's, the second if nothing else is there */
     const bool mid2 = binned && fork && nsplit == 0 && most(UF_CHUNK) == 0 && most(UF_BIG) > 0;
-    hipStream_t sm = mid2 ? c->st2 : binned && fork && wvs > 0 && most(UF_BIG) > 0 ? sw : c->st;
+    hipStream_t sb = chunk1 && wvs > 0 ? sw : c->st;
+    hipStream_t sm = mid2 ? c->st2 : (chunk1 || (binned && fork && most(UF_BIG) > 0)) && wvs > 0 ? sw : c->st;
     if (wvs > 0 && fork) hipStreamWaitEvent(sw, c->ev_s0, 0);
     if (mid2) hipStreamWaitEvent(c->st2, c->ev_s0, 0);
-    if (sm == c->st && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, c->st);
+    if (sm == sb && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, sb);
     if (most(UF_MID) > 0) AHF_UNBIND_LAUNCH(UF_MID, q0[UF_WAVE], most(UF_MID), AHF_BLOCK, 8, 2, sm);
     if (mid2) hipEventRecord(c->ev_s1, c->st2);
     if (wvs > 0) {
@@ -3299,8 +3384,8 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
       }
       if (fork) hipEventRecord(c->ev_s2, sw);
     }
-    if (sm != c->st && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, c->st);
-    if (fork && (mid2 || most(UF_CHUNK) > 0)) hipStreamWaitEvent(c->st, c->ev_s1, 0);
+    if (sm != sb && most(UF_BIG) > 0) AHF_UNBIND_LAUNCH(UF_BIG, q0[UF_MID], most(UF_BIG), AHF_BIG_BLOCK, 8, 1, sb);
+    if (fork && (mid2 || chunk2)) hipStreamWaitEvent(c->st, c->ev_s1, 0);
     if (fork && wvs > 0) hipStreamWaitEvent(c->st, c->ev_s2, 0);
 #undef AHF_UNBIND_LAUNCH
     if (nsplit > 0) {

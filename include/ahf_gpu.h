@@ -194,9 +194,8 @@ int ahfgpu_unbind(ahfgpu_ctx *ctx, const ahfgpu_unbind_params *p, int mode, doub
  * min_members members (and NminPerHalo) are unbound on a second path that
  * runs their passes over the members as flat kernels over all such haloes
  * and keeps one workgroup per halo only for the recurrence; the others stay
- * in the persistent kernels.  0 restores the default (4097 once a halo has
- * 16384, else none), a negative value sends every halo to the persistent
- * kernels.  Both paths give the
+ * in the persistent kernels.  0 restores the default (16384), a negative
+ * value sends every halo to the persistent kernels.  Both paths give the
  * same members and fields. */
 int ahfgpu_set_unbind_split(ahfgpu_ctx *ctx, int64_t min_members);
 
@@ -313,7 +312,7 @@ int ahfgpu_gridinfo_results(ahfgpu_ctx *ctx, int grid, int32_t *colour, int32_t 
  * schedule.json beside the library's directory (written by the autotuner,
  * python -m ahf_amd.autotune), when it exists. */
 typedef struct {
-  int64_t split_min;   /* haloes of this many members or more take the split path (-1: none); 4097, once a halo has 16384 */
+  int64_t split_min;   /* haloes of this many members or more take the split path (-1: none); 16384 */
   int64_t prof_split;  /* HaloProfiles: haloes of this many members or more on four wavefronts (-1: none); 2048 */
   int64_t big_halo;    /* unbinding: haloes of this many members or more on 512-thread workgroups; 2049 (at most) */
   int64_t wave_halo;   /* unbinding: haloes below this many members on one wavefront; 513 (at most) */
