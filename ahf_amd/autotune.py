@@ -43,7 +43,7 @@ CANDIDATES = {
     "graph_batch": [4, 2, 8],
     "split_spec": [3, 1, 2, 4, 6, -1],
     "prof_split": [2048, 512, 1024, 4096, 8192],
-    "prof_tiled": [32768, 8192, 16384, 65536, 131072, -1],
+    "prof_tiled": [0, 4096, 16384, 32768, 65536, 131072, -1],
 }
 # which timing decides each field
 DECIDES = {"kmax_big": "amr", "kmax_small": "amr", "march_zn": "amr", "big_halo": "unbind", "wave_halo": "unbind",

@@ -506,7 +506,17 @@ __device__ void prf_radii(const ProfConst &K, int64_t n, const uint32_t *__restr
  * that decrease keep the sequential walk.
  */
 #define PRF_TILE 1024
-#define AHF_PROF_TILED 32768
+/* the default prof_tiled.  A member costs a lane's chain of additions some 10
+ * ns there, k_profiles<4> some 30 ns (one workgroup's barriers), and the
+ * longest walk is what the call waits for: from 32768 on instead of 8192, the
+ * profiles of a 128^3 catalogue took 1.1 to 1.2 ms for 0.72 to 0.90, of a
+ * 256^3 one with haloes of 8000 0.67 for 0.43, of 20,000 haloes 1.38 for 0.76
+ * where none was larger; from 4096 on nothing more.  The rows take 164 bytes a
+ * member: haloes below AHF_PROF_TILED_ANY only while all of them together have
+ * at most AHF_PROF_TILED_SUM. */
+#define AHF_PROF_TILED 8192
+#define AHF_PROF_TILED_ANY 32768
+#define AHF_PROF_TILED_SUM ((int64_t)1 << 25)
 
 struct PrfTiled {
   int64_t h, n, P, to; /* halo, members, members the walk reaches, offset in the tiled scratch */
@@ -1991,7 +2001,8 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
   int64_t Nt = 0;
   for (int32_t h : bigl) {
     const int64_t n = hn[(size_t)h];
-    if (n < tiled) continue;
+    /* largest first: the haloes walked over the device are the list's first */
+    if (n < tiled || (c->prof_tiled == 0 && n < AHF_PROF_TILED_ANY && Nt + n > AHF_PROF_TILED_SUM)) break;
     if (tmap_h.empty()) tmap_h.assign((size_t)nh, -1);
     PrfTiled T;
     memset(&T, 0, sizeof(T));
@@ -2114,11 +2125,18 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
       if (nbig > ntl) big_launch(ntl ? c->st : c->st2, ntl, nbig - ntl);
       hipEventRecord(c->ev_s1, c->st2);
     }
-    hipLaunchKernelGGL(k_profiles<1>, dim3((unsigned)nh), dim3(64), 0, c->st, K, s->off, s->order, big, out, d_pr,
+    /* the small haloes: behind the peaks on the third stream where the first
+     * has big ones to walk */
+    hipStream_t s1 = ntl && nbig > ntl ? c->st3 : c->st;
+    hipLaunchKernelGGL(k_profiles<1>, dim3((unsigned)nh), dim3(64), 0, s1, K, s->off, s->order, big, out, d_pr,
                        s->ip_in, s->buf_a, s->buf_b, s->cen, d_nb, d_pofs, c->px, c->py, c->pz, c->vx, c->vy, c->vz,
                        sc, sc + ne, sc + 2 * ne, r->props, r->prof, (const PrfTiled *)nullptr,
                        (const int32_t *)nullptr, c->pv);
     if (nbig) hipStreamWaitEvent(c->st, c->ev_s1, 0);
+    if (s1 != c->st) {
+      hipEventRecord(c->ev_s2, s1);
+      hipStreamWaitEvent(c->st, c->ev_s2, 0);
+    }
     c->timer_end(e0, TIMER_PROFILES, 0.0);
   }
   c->timers_reset(TIMER_PROFILES, TIMER_PROFILES);

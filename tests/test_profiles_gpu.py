@@ -116,6 +116,34 @@ def test_profiles_of_given_haloes(oracle, snapgen, ctx, tmp_path, cfg, side, see
     _compare(ref, nb, props, prof, f"cfg{cfg}/{side}/g{gather}/split{split}")
 
 
+@pytest.mark.parametrize("sizes", [(8191,), (8192,), (8193, 8191, 300), (12000, 8192, 2048, 2047, 40)])
+def test_profiles_walk_line(ctx, sizes):
+    """haloes on both sides of the size from which they are walked over the
+    device give the bits of the walk on one workgroup, with other big and
+    small haloes beside them"""
+    rng = np.random.default_rng(sum(sizes))
+    n = sum(sizes)
+    centre = rng.random((len(sizes), 3))
+    d = np.concatenate([0.02 * np.sort(rng.random(k))[:, None] * (lambda v: v / np.linalg.norm(v, axis=1)[:, None])(
+        rng.standard_normal((k, 3))) for k in sizes])
+    pos = ((np.repeat(centre, sizes, axis=0) + d) % 1.0).astype(np.float32)
+    pos[pos >= 1.0] = 0.0
+    ctx.set_particles(pos, rng.standard_normal((n, 3)).astype(np.float32))
+    pr = np.stack([np.full(len(sizes), 3.0e3), np.full(len(sizes), 0.02)], axis=1)
+    got = []
+    try:
+        for tiled in (0, -1):
+            ctx.set_schedule(prof_tiled=tiled)
+            ctx.set_halos(centre, np.array(sizes, np.int64), np.arange(n, dtype=np.uint64))
+            got.append(ctx.halo_profiles(20, 1.0, 1.0, 1.0, 1.0, 0.1, phi0_rvir=pr))
+    finally:
+        _reset_split(ctx)
+    (nb, props, prof), (nb1, props1, prof1) = got
+    assert np.array_equal(nb, nb1) and int(nb.min()) > 0
+    assert np.array_equal(props, props1, equal_nan=True)
+    assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(prof, prof1))
+
+
 @pytest.mark.parametrize("cfg,side,seed,gather", [(2, 800, 1002, 0), (3, 48, 5, 0), (2, 400, 1002, 1)])
 def test_profiles_end_to_end(oracle, snapgen, ctx, tmp_path, cfg, side, seed, gather):
     """construction and profiles on the GPU, against the oracle's dump"""
