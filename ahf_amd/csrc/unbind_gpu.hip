@@ -47,6 +47,7 @@
 #include "gpu_ctx.h"
 #include "halo_set.h"
 #include "nr_order.h"
+#include "unbind_core.h"
 
 using namespace ahf;
 
@@ -1423,9 +1424,12 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
      * members in order with the bulk velocity that it has just changed; a
      * wavefront evaluates its members again, with the totals of its lower
      * lanes' last statuses, until none changes; the wavefronts then hand up
-     * their totals, until no total changes.  Every evaluation settles at
-     * least one thread more and every hand-over one wavefront more, and what
-     * no longer changes is the sequential answer.  (Whole-list sweeps with
+     * their totals, until no status has changed since the totals before.
+     * Every evaluation settles at least one thread more and every hand-over
+     * one wavefront more, and what no longer changes is the sequential
+     * answer.  Statuses are compared and not totals: a member with a NaN
+     * velocity stays bound, as in AHF, and its total is never equal to
+     * itself.  (Whole-list sweeps with
      * the statuses of the sweep before settle one member at a time where
      * statuses near the centre hang on each other: 1.9 ms for the haloes of
      * 513 to 2048 members of 20,000, where this takes 0.11.)
@@ -1434,7 +1438,7 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
      */
     uint32_t bj = alive, ub = 0;
     const int w = t >> 6;
-    D4 base = {seed.x, seed.y, seed.z, 1.0}, mine = {0, 0, 0, 0};
+    D4 base = {seed.x, seed.y, seed.z, 1.0};
     auto sums = [&]() {
       /* the velocities are converted in every evaluation: kept as doubles
        * from one to the next (the compiler would) they do not fit */
@@ -1455,12 +1459,13 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
     if constexpr (NW > 1) {
       D4 inc, ex;
       wave_scan4_dpp(sums(), &inc, &ex);
-      mine = res_top4(inc);
-      if ((t & 63) == 0) S.tot[0][w] = mine;
+      const D4 all = res_top4(inc);
+      if ((t & 63) == 0) S.tot[0][w] = all;
       __syncthreads();
       for (int k = 0; k < w; k++) base = add4(base, S.tot[0][k]);
     }
     for (int round = 1;; round++) {
+      const uint32_t was = bj;
       D4 inc, ex;
       for (;;) {
         sweeps++;
@@ -1503,11 +1508,10 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
       }
       if constexpr (NW == 1) break;
       const D4 now = res_top4(inc);
-      const int moved = now.x != mine.x || now.y != mine.y || now.z != mine.z || now.m != mine.m;
-      mine = now;
+      const uint64_t moved = __ballot(ahf_handup_moved(was, bj));
       if ((t & 63) == 0) {
         S.tot[round & 1][w] = now;
-        S.moved[round & 1][w] = moved;
+        S.moved[round & 1][w] = moved != 0ull;
       }
       __syncthreads();
       int any = 0;

@@ -78,6 +78,18 @@ def test_heavy_block_sum(tmp_path):
         assert r.returncode == 0, r.stderr[-2000:] + r.stdout
 
 
+def test_handup_ends(tmp_path):
+    """the register form's hand-up between wavefronts ends, with the
+    sequential loop's statuses, whatever the velocities: NaN, infinities and
+    very large values in the first, a middle and the last wavefront"""
+    exe = str(tmp_path / "handup_check")
+    subprocess.run(["gcc", "-std=c11", "-O2", "-ffp-contract=off", "-Wno-unused-function", "-o", exe,
+                    os.path.join(HERE, "emu", "handup_check.c"), "-lm"], check=True)
+    for seed in (1, 2):
+        r = subprocess.run([exe, "2000", str(seed)], capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:] + r.stdout
+
+
 def test_fold64_replay(tmp_path):
     """an FP64 running-sum fold (integer steps on a binade's grid,
     exact ties by parity, plain steps across binades and from zero or

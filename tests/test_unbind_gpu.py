@@ -296,6 +296,57 @@ def test_form_sizes(oracle, ctx, tmp_path, cuts, plain, split, band, sched):
         assert np.array_equal(ref.ovdens, props[:, 3])
 
 
+ODD = [(n, where, value) for n in (300, 600, 2000, 4000, 5000) for where in ("first", "middle", "last")
+       for value in ("nan", "inf", "both")]
+
+
+def _odd_snapshot(path, seed):
+    """isolated haloes whose first, a middle or last wavefront of members holds
+    a NaN velocity, one infinite velocity, or a NaN and behind it infinities of
+    both signs; none among the members that the first seed is chosen from"""
+    rng = np.random.default_rng(seed)
+    pos, mom, lists, cen, n0 = [], [], [], [], 0
+    for n, where, value in ODD:
+        c = np.float32(rng.uniform(0.05, 0.95, 3)).astype(np.float64)
+        d = rng.normal(size=(n, 3))
+        p = (c + (0.01 * rng.random(n) ** 1.5)[:, None] * d / np.linalg.norm(d, axis=1)[:, None]).astype(np.float32)
+        o = np.argsort(((p.astype(np.float64) - c) ** 2).sum(1))
+        v = rng.normal(0.0, 1.0, (n, 3)) * np.sqrt(n) * 2e-3 + rng.normal(0.0, 3.0, 3)
+        v[rng.random(n) < 0.15] *= 3.0
+        at = {"first": min(100, n // 3), "middle": n // 2, "last": n - 15}[where]
+        if value != "inf":
+            v[o[at], 1] = np.nan
+        if value != "nan":
+            v[o[at + 3], 0] = np.inf
+        if value == "both":
+            v[o[at + 5], 0] = -np.inf
+        pos.append(p)
+        mom.append(v)
+        lists.append((rng.permutation(n) + n0).astype(np.uint64))
+        cen.append(c)
+        n0 += n
+    dumps.write_snapshot(path, np.concatenate(pos), np.concatenate(mom), boxsize=1.0, pmass=1e8, L_dom=16,
+                         centres=np.array(cen), halo_lists=lists, r_fac=1.0, v_fac=1.0, phi_fac=2e-7, hubble=10.0,
+                         ovlim=60.0, rho_vir=6e13, gather_rad=np.full(len(lists), 0.02))
+
+
+@pytest.mark.parametrize("cuts,plain", [(0, 0), (WITH_RVIR, 0), (0, 1), (WITH_RVIR, 1)])
+def test_odd_velocities(oracle, ctx, tmp_path, cuts, plain):
+    """a NaN velocity stays bound and an infinite one does not, as in AHF, and
+    the rounds of the unbinding end, in every form up to the chunked one"""
+    snap, out = str(tmp_path / "n.snap"), str(tmp_path / "o.halo")
+    _odd_snapshot(snap, 3)
+    dump = oracle.oracle_construct_dump if cuts else oracle.oracle_unbind_dump
+    assert dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    s = dumps.read_snapshot(snap)
+    nan = np.array([np.isnan(s.mom[m.astype(np.int64)]).any() for m in ref.ipart])
+    assert np.array_equal(nan, [value != "inf" for _, _, value in ODD]) and np.all(ref.npart < s.halo_npart)
+    print(f"[odd] cuts {cuts} plain {plain}: {s.nhalos} haloes", flush=True)
+    _, (npart, props, lists) = _construct_gpu(ctx, s, plain | cuts, split=-1) if cuts else _run_gpu(ctx, s, plain, split=-1)
+    _compare(ref, npart, props, lists, f"odd velocities {cuts} {plain}")
+
+
 def _edge_halo(rng, n, phi_fac, vtune2, minpart):
     """positions (offsets) and velocities of a halo in radial order, one of
     whose members sits within about one unit of rounding of the bound test as
