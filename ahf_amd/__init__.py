@@ -132,6 +132,7 @@ def load():
     lib.ahfgpu_set_profile_split.argtypes = [P, ctypes.c_int64]
     lib.ahfgpu_set_schedule.argtypes = [P, ctypes.POINTER(Schedule)]
     lib.ahfgpu_get_schedule.argtypes = [P, ctypes.POINTER(Schedule)]
+    lib.ahfgpu_set_memory_limit.argtypes = [P, ctypes.c_uint64]
     lib.ahfgpu_set_timing.argtypes = [P, ctypes.c_int]
     lib.ahfgpu_gridinfo.argtypes = [P, ctypes.POINTER(GridinfoParams), ctypes.POINTER(GridinfoInfo)]
     lib.ahfgpu_gridinfo_results.argtypes = [P, ctypes.c_int, P, P]
@@ -198,6 +199,10 @@ class Context:
         for k, v in fields.items():
             setattr(sc, k, int(v))
         self._check(self.lib.ahfgpu_set_schedule(self.h, ctypes.byref(sc)))
+
+    def set_memory_limit(self, nbytes):
+        """the most device memory each work area hands out at a time (0: no limit)"""
+        self._check(self.lib.ahfgpu_set_memory_limit(self.h, int(nbytes)))
 
     def set_gather_mode(self, mode):
         """deposit kernel choice (same results in every mode)"""

@@ -2778,16 +2778,11 @@ static int final_lists(ahfgpu_ctx *c, int lev, int64_t *list0, uint32_t *list)
   if (hipSetDevice(c->device) != hipSuccess) return c->fail(AHFGPU_EHIP, "hipSetDevice");
   /* the scratch lies behind the hierarchy and is given back at once */
   Arena &A = c->arena;
-  const size_t cur = A.cur, used = cur < A.chunks.size() ? A.chunks[cur].used : 0;
   struct Rewind {
     Arena &A;
-    size_t cur, used;
-    ~Rewind()
-    {
-      for (size_t k = cur; k < A.chunks.size(); k++) A.chunks[k].used = k == cur ? used : 0;
-      A.cur = cur;
-    }
-  } rewind{A, cur, used};
+    Arena::Mark m;
+    ~Rewind() { A.rewind(m); }
+  } rewind{A, A.mark()};
   const bool ranked = l.child != nullptr;
   int64_t *d0 = A.get<int64_t>(nn + 1), *cnt = nullptr, *rbx = nullptr, *rtmp = nullptr;
   uint32_t *dl = list ? A.get<uint32_t>(nl) : nullptr, *rank = nullptr, *tmp = nullptr;

@@ -116,6 +116,13 @@ extern "C" int ahfgpu_set_schedule(ahfgpu_ctx *c, const ahfgpu_schedule *s)
   return 0;
 }
 
+extern "C" int ahfgpu_set_memory_limit(ahfgpu_ctx *c, uint64_t bytes)
+{
+  if (!c) return AHFGPU_EINVAL;
+  c->arena.limit = c->uarena.limit = c->parena.limit = c->garena.limit = (size_t)bytes;
+  return 0;
+}
+
 extern "C" int ahfgpu_get_schedule(ahfgpu_ctx *c, ahfgpu_schedule *s)
 {
   if (!c || !s) return AHFGPU_EINVAL;

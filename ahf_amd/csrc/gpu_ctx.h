@@ -29,16 +29,34 @@ struct Arena {
   std::vector<Chunk> chunks;
   size_t cur = 0;
   size_t min_chunk = (size_t)256 << 20;
+  size_t limit = 0; /* most bytes handed out at a time (0: what the device has) */
 
   void reset()
   {
     for (auto &c : chunks) c.used = 0;
     cur = 0;
   }
+  size_t taken() const
+  {
+    size_t n = 0;
+    for (const auto &c : chunks) n += c.used;
+    return n;
+  }
+  /* what is handed out from a mark on is given back by rewind() */
+  struct Mark {
+    size_t cur, used;
+  };
+  Mark mark() const { return Mark{cur, cur < chunks.size() ? chunks[cur].used : 0}; }
+  void rewind(Mark m)
+  {
+    for (size_t k = m.cur; k < chunks.size(); k++) chunks[k].used = k == m.cur ? m.used : 0;
+    cur = m.cur;
+  }
   void *raw(size_t bytes)
   {
     bytes = (bytes + 255) & ~(size_t)255;
     if (bytes == 0) bytes = 256;
+    if (limit && taken() + bytes > limit) return nullptr;
     while (cur < chunks.size()) {
       Chunk &c = chunks[cur];
       if (c.size - c.used >= bytes) {

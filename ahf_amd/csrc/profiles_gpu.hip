@@ -513,7 +513,7 @@ __device__ void prf_radii(const ProfConst &K, int64_t n, const uint32_t *__restr
  * 256^3 one with haloes of 8000 0.67 for 0.43, of 20,000 haloes 1.38 for 0.76
  * where none was larger; from 4096 on nothing more.  The rows take 164 bytes a
  * member: haloes below AHF_PROF_TILED_ANY only while all of them together have
- * at most AHF_PROF_TILED_SUM. */
+ * at most AHF_PROF_TILED_SUM, and only where the device has room for the rows. */
 #define AHF_PROF_TILED 8192
 #define AHF_PROF_TILED_ANY 32768
 #define AHF_PROF_TILED_SUM ((int64_t)1 << 25)
@@ -1998,25 +1998,32 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
   std::vector<PrfTiled> htl;
   std::vector<PrfTile> htile;
   std::vector<int32_t> tmap_h;
-  int64_t Nt = 0;
-  for (int32_t h : bigl) {
-    const int64_t n = hn[(size_t)h];
-    /* largest first: the haloes walked over the device are the list's first */
-    if (n < tiled || (c->prof_tiled == 0 && n < AHF_PROF_TILED_ANY && Nt + n > AHF_PROF_TILED_SUM)) break;
-    if (tmap_h.empty()) tmap_h.assign((size_t)nh, -1);
-    PrfTiled T;
-    memset(&T, 0, sizeof(T));
-    T.h = h;
-    T.n = n;
-    T.to = Nt;
-    T.t0 = (int32_t)htile.size();
-    for (int64_t j0 = 0; j0 < n; j0 += PRF_TILE) htile.push_back(PrfTile{(int32_t)htl.size(), 0, j0});
-    T.t1 = (int32_t)htile.size();
-    tmap_h[(size_t)h] = (int32_t)htl.size();
-    htl.push_back(T);
-    Nt += n + (n & 1); /* rows at even offsets: member pairs are 16-byte aligned */
-  }
-  const int64_t ntl = (int64_t)htl.size(), ntile = (int64_t)htile.size();
+  int64_t Nt = 0, ntl = 0, ntile = 0;
+  auto lay_out = [&](int64_t least) {
+    htl.clear();
+    htile.clear();
+    tmap_h.clear();
+    Nt = 0;
+    for (int32_t h : bigl) {
+      const int64_t n = hn[(size_t)h];
+      /* largest first: the haloes walked over the device are the list's first */
+      if (n < least || (c->prof_tiled == 0 && n < AHF_PROF_TILED_ANY && Nt + n > AHF_PROF_TILED_SUM)) break;
+      if (tmap_h.empty()) tmap_h.assign((size_t)nh, -1);
+      PrfTiled T;
+      memset(&T, 0, sizeof(T));
+      T.h = h;
+      T.n = n;
+      T.to = Nt;
+      T.t0 = (int32_t)htile.size();
+      for (int64_t j0 = 0; j0 < n; j0 += PRF_TILE) htile.push_back(PrfTile{(int32_t)htl.size(), 0, j0});
+      T.t1 = (int32_t)htile.size();
+      tmap_h[(size_t)h] = (int32_t)htl.size();
+      htl.push_back(T);
+      Nt += n + (n & 1); /* rows at even offsets: member pairs are 16-byte aligned */
+    }
+    ntl = (int64_t)htl.size();
+    ntile = (int64_t)htile.size();
+  };
   PrfTiled *d_tl = nullptr;
   PrfTile *d_tile = nullptr;
   int32_t *d_tmap = nullptr, *tcmax = nullptr;
@@ -2026,7 +2033,10 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
   PrfChain *d_chains = nullptr;
   PrfRows R;
   memset(&R, 0, sizeof(R));
-  if (ntl) {
+  double *d_props = A.get<double>(nh * PP_N), *d_prof = A.get<double>(tot * PQ_N);
+  if (!d_props || !d_prof || (nbig && !d_big)) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (profiles)");
+  auto get_rows = [&]() {
+    if (ntl == 0) return true;
     d_tl = A.get<PrfTiled>(ntl);
     d_tile = A.get<PrfTile>(ntile);
     d_tmap = A.get<int32_t>(nh);
@@ -2042,7 +2052,7 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
     int32_t *irows = A.get<int32_t>(3 * Nt);
     if (!d_tl || !d_tile || !d_tmap || !tcmax || !tflmax || !tmb || !tEmin || !tpv || !tpi || !tib || !d_chains ||
         !rows || !irows)
-      return c->fail(AHFGPU_ENOMEM, "device arena exhausted (profiles over the device)");
+      return false;
     double *w = rows;
     auto take = [&]() { double *r = w; w += Nt; return r; };
     R.dd = take(); R.gx = take(); R.gy = take(); R.gz = take();
@@ -2050,14 +2060,24 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
     R.tt = take(); R.phi = take(); R.phir = take();
     for (int k = 0; k < 6; k++) R.ine[k] = take();
     R.c = irows; R.bp = irows + Nt; R.bi = irows + 2 * Nt;
+    return true;
+  };
+  lay_out(tiled);
+  const Arena::Mark behind = A.mark();
+  bool got = get_rows();
+  if (!got && c->prof_tiled == 0) {
+    /* no room for the rows of haloes that a workgroup walks without any */
+    A.rewind(behind);
+    lay_out(AHF_PROF_TILED_ANY);
+    got = get_rows();
   }
+  if (!got) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (profiles over the device)");
   ProfResult *r = (ProfResult *)c->prof_result;
   if (!r) c->prof_result = r = new ProfResult();
   r->nh = nh;
   r->nbins_tot = tot;
-  r->props = A.get<double>(nh * PP_N);
-  r->prof = A.get<double>(tot * PQ_N);
-  if (!r->props || !r->prof || (nbig && !d_big)) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (profiles)");
+  r->props = d_props;
+  r->prof = d_prof;
   if (nh) {
     hipMemcpyAsync(d_nb, nb.data(), (size_t)nh * 4, hipMemcpyHostToDevice, c->st);
     hipMemcpyAsync(d_pofs, pofs.data(), (size_t)nh * 8, hipMemcpyHostToDevice, c->st);

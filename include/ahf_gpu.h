@@ -330,6 +330,13 @@ typedef struct {
 int ahfgpu_set_schedule(ahfgpu_ctx *ctx, const ahfgpu_schedule *s);
 int ahfgpu_get_schedule(ahfgpu_ctx *ctx, ahfgpu_schedule *s);
 
+/* No counterpart in the reference: the most device memory that each of the
+ * context's work areas (hierarchy, unbinding, profiles, isolated refinements)
+ * may hand out at a time, for a process that shares its GPU; 0, the default:
+ * what the device has.  Calls that need more return AHFGPU_ENOMEM, as they do
+ * when the device is full, or take the form that does with less. */
+int ahfgpu_set_memory_limit(ahfgpu_ctx *ctx, uint64_t bytes);
+
 /* No counterpart in the reference: the stage timers (HIP events around
  * each stage, read by ahfgpu_last_timing and ahfgpu_timer_get) on (1, the
  * default) or off (0: the timings read 0), for callers that make many

@@ -116,11 +116,9 @@ def test_profiles_of_given_haloes(oracle, snapgen, ctx, tmp_path, cfg, side, see
     _compare(ref, nb, props, prof, f"cfg{cfg}/{side}/g{gather}/split{split}")
 
 
-@pytest.mark.parametrize("sizes", [(8191,), (8192,), (8193, 8191, 300), (12000, 8192, 2048, 2047, 40)])
-def test_profiles_walk_line(ctx, sizes):
-    """haloes on both sides of the size from which they are walked over the
-    device give the bits of the walk on one workgroup, with other big and
-    small haloes beside them"""
+def _given_haloes(ctx, sizes):
+    """haloes of these sizes as the context's particles; their centres and
+    member indices, and (Phi0, R_vir)"""
     rng = np.random.default_rng(sum(sizes))
     n = sum(sizes)
     centre = rng.random((len(sizes), 3))
@@ -129,19 +127,59 @@ def test_profiles_walk_line(ctx, sizes):
     pos = ((np.repeat(centre, sizes, axis=0) + d) % 1.0).astype(np.float32)
     pos[pos >= 1.0] = 0.0
     ctx.set_particles(pos, rng.standard_normal((n, 3)).astype(np.float32))
-    pr = np.stack([np.full(len(sizes), 3.0e3), np.full(len(sizes), 0.02)], axis=1)
+    return centre, np.arange(n, dtype=np.uint64), np.stack([np.full(len(sizes), 3.0e3), np.full(len(sizes), 0.02)], axis=1)
+
+
+def _same_profiles(a, b):
+    (nb, props, prof), (nb1, props1, prof1) = a, b
+    assert np.array_equal(nb, nb1) and int(nb.min()) > 0
+    assert np.array_equal(props, props1, equal_nan=True)
+    assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(prof, prof1))
+
+
+@pytest.mark.parametrize("sizes", [(8191,), (8192,), (8193, 8191, 300), (12000, 8192, 2048, 2047, 40)])
+def test_profiles_walk_line(ctx, sizes):
+    """haloes on both sides of the size from which they are walked over the
+    device give the bits of the walk on one workgroup, with other big and
+    small haloes beside them"""
+    centre, ip, pr = _given_haloes(ctx, sizes)
     got = []
     try:
         for tiled in (0, -1):
             ctx.set_schedule(prof_tiled=tiled)
-            ctx.set_halos(centre, np.array(sizes, np.int64), np.arange(n, dtype=np.uint64))
+            ctx.set_halos(centre, np.array(sizes, np.int64), ip)
             got.append(ctx.halo_profiles(20, 1.0, 1.0, 1.0, 1.0, 0.1, phi0_rvir=pr))
     finally:
         _reset_split(ctx)
-    (nb, props, prof), (nb1, props1, prof1) = got
-    assert np.array_equal(nb, nb1) and int(nb.min()) > 0
-    assert np.array_equal(props, props1, equal_nan=True)
-    assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(prof, prof1))
+    _same_profiles(*got)
+
+
+@pytest.mark.parametrize("sizes,fits", [((32767, 8192, 300), 0), ((40000, 32767, 8192, 300), 40000), ((40000, 300), None)])
+def test_profiles_without_room(ctx, sizes, fits):
+    """haloes below 32768 members do without the rows of the walk over the
+    device where there is no room for them, and give the same bits; the larger
+    ones need theirs"""
+    import ahf_amd
+    centre, ip, pr = _given_haloes(ctx, sizes)
+    args = (20, 1.0, 1.0, 1.0, 1.0, 0.1)
+    ctx.set_halos(centre, np.array(sizes, np.int64), ip)
+    ref = ctx.halo_profiles(*args, phi0_rvir=pr)
+    try:
+        # 24 bytes a member for every call, 164 for each one that has rows; the
+        # haloes' records and the tiles' take less than the 400,000 beside them
+        ctx.set_memory_limit(24 * sum(sizes) + 164 * (fits or 0) + 400000)
+        if fits is None:
+            with pytest.raises(ahf_amd.AhfGpuError):
+                ctx.halo_profiles(*args, phi0_rvir=pr)
+        else:
+            _same_profiles(ctx.halo_profiles(*args, phi0_rvir=pr), ref)
+        ctx.set_schedule(prof_tiled=8192)
+        with pytest.raises(ahf_amd.AhfGpuError):
+            ctx.halo_profiles(*args, phi0_rvir=pr)
+    finally:
+        ctx.set_memory_limit(0)
+        _reset_split(ctx)
+    _same_profiles(ctx.halo_profiles(*args, phi0_rvir=pr), ref)
 
 
 @pytest.mark.parametrize("cfg,side,seed,gather", [(2, 800, 1002, 0), (3, 48, 5, 0), (2, 400, 1002, 1)])
