@@ -1327,7 +1327,8 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
     if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0); /* the loads of four members in flight */
   }
   /* the sums of |v| that bound the rounding of the bulk-velocity sums: over
-   * the whole list, so no smaller than over the members still bound */
+   * the whole list, so no smaller than over the members still bound; made
+   * again behind an iteration that needed the exact tests */
   {
     D4 asum;
     (void)res_scan4<BS>(av, &asum, S);
@@ -1550,6 +1551,18 @@ __device__ __forceinline__ void unbind_resident(const UnbindConst &K, int64_t n0
         r++;
       }
       __syncthreads();
+      /* a member that has just left, if fast enough, would make all later
+       * iterations uncertain */
+      D4 vs = {0, 0, 0, 0}, asum;
+#pragma unroll
+      for (int i = 0; i < IPT; i++)
+        if ((bj >> i) & 1u) {
+          vs.x += fabs((double)vx[i]);
+          vs.y += fabs((double)vy[i]);
+          vs.z += fabs((double)vz[i]);
+        }
+      (void)res_scan4<BS>(vs, &asum, S);
+      if (t == 0) S.asum = asum;
     }
     alive = bj;
     const int before = n;

@@ -347,6 +347,45 @@ def test_odd_velocities(oracle, ctx, tmp_path, cuts, plain):
     _compare(ref, npart, props, lists, f"odd velocities {cuts} {plain}")
 
 
+FAST = [60, 130, 400, 700, 1800, 3000, 4000, 6000]
+
+
+def _fast_snapshot(path, seed):
+    """isolated haloes with one member of 10^25 times the others' speed, which
+    leaves in the first iteration"""
+    rng = np.random.default_rng(seed)
+    pos, mom, lists, cen, n0 = [], [], [], [], 0
+    for n in FAST:
+        c = np.float32(rng.uniform(0.05, 0.95, 3)).astype(np.float64)
+        d = rng.normal(size=(n, 3))
+        p = (c + (0.01 * rng.random(n) ** 1.5)[:, None] * d / np.linalg.norm(d, axis=1)[:, None]).astype(np.float32)
+        o = np.argsort(((p.astype(np.float64) - c) ** 2).sum(1))
+        v = rng.normal(0.0, 1.0, (n, 3)) * np.sqrt(n) * 2e-3
+        v[o[20 + np.flatnonzero(rng.random(n - 20) < 0.15)]] *= 3.0
+        v[o[n // 2]] = [1e25, 0.0, -1e25]
+        pos.append(p)
+        mom.append(v)
+        lists.append((rng.permutation(n) + n0).astype(np.uint64))
+        cen.append(c)
+        n0 += n
+    dumps.write_snapshot(path, np.concatenate(pos), np.concatenate(mom), boxsize=1.0, pmass=1e8, L_dom=16,
+                         centres=np.array(cen), halo_lists=lists, r_fac=1.0, v_fac=1.0, phi_fac=2e-7, hubble=10.0,
+                         ovlim=60.0, rho_vir=6e13, gather_rad=np.full(len(lists), 0.02))
+
+
+@pytest.mark.parametrize("plain", [0, 1])
+def test_fast_member_widens_one_iteration(oracle, ctx, tmp_path, plain):
+    """a member too fast for the rounding bound makes the iteration that removes
+    it uncertain, in every form, and none of the later ones"""
+    snap, out = str(tmp_path / "v.snap"), str(tmp_path / "o.halo")
+    _fast_snapshot(snap, 4)
+    assert oracle.oracle_unbind_dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    info, (npart, props, lists) = _run_gpu(ctx, dumps.read_snapshot(snap), plain, split=-1)
+    _compare(ref, npart, props, lists, f"fast member {plain}")
+    assert props[:, 4].min() >= 2 and info.n_exact_replays == len(FAST)
+
+
 def _edge_halo(rng, n, phi_fac, vtune2, minpart):
     """positions (offsets) and velocities of a halo in radial order, one of
     whose members sits within about one unit of rounding of the bound test as
