@@ -34,6 +34,35 @@ def fuzz_snapshot(path, seed, non_pow2=False):
     return dict(L=L, n=len(pos), Nth_dom=nth, Nth_ref=nref, L_max=Lmax)
 
 
+def short_haloes_snapshot(path, seed, nh):
+    """nh isolated haloes of 20 to 600 members, among them both sides of 128
+    and of 512, with outskirts below the overdensity limit and velocities with
+    a tail above the escape speed.  Returns, per halo, the members that the cut
+    ahead of the unbinding leaves."""
+    rng = np.random.default_rng(seed)
+    sizes = np.exp(rng.uniform(np.log(20), np.log(600), nh)).astype(np.int64)
+    sizes[:60] = np.resize([20, 127, 128, 129, 511, 512, 513, 600], 60)
+    n = int(sizes.sum())
+    cen = np.float32(rng.uniform(0.05, 0.95, (nh, 3))).astype(np.float64)
+    d = rng.standard_normal((n, 3))
+    r = 0.01 * rng.random(n) ** 1.5
+    pos = (np.repeat(cen, sizes, axis=0) + r[:, None] * d / np.linalg.norm(d, axis=1)[:, None]).astype(np.float32)
+    mom = rng.standard_normal((n, 3)) * np.repeat(np.sqrt(sizes) * 2e-3, sizes)[:, None]
+    mom[rng.random(n) < 0.15] *= 3.0
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    lists = [(off[h] + rng.permutation(sizes[h])).astype(np.uint64) for h in range(nh)]
+    ovlim, rho_vir, pmass = 200.0, 3e13, 1e8
+    dumps.write_snapshot(path, pos, mom, boxsize=1.0, pmass=pmass, L_dom=16, centres=cen, halo_lists=lists, r_fac=1.0,
+                         v_fac=1.0, phi_fac=2e-7, hubble=10.0, ovlim=ovlim, rho_vir=rho_vir, gather_rad=np.full(nh, 0.02))
+    dist = np.sqrt(((pos.astype(np.float64) - np.repeat(cen, sizes, axis=0)) ** 2).sum(1))
+    left = np.zeros(nh, np.int64)
+    for h in range(nh):
+        x = np.sort(dist[off[h]:off[h + 1]])
+        low = np.flatnonzero(np.arange(1, len(x) + 1) * pmass < ovlim * rho_vir * (4 * np.pi / 3 * x ** 3))
+        left[h] = low[0] + 1 if len(low) else len(x)
+    return left
+
+
 # HaloProfiles comparisons: exact where the inputs fix the bits
 # values computed from the bin radii or through log(): device libm
 LIBM_BINS = {"r", "ovdens", "dens", "v2_circ"}

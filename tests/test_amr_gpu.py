@@ -129,6 +129,27 @@ def test_final_lists(oracle, ctx, tmp_path, seed):
         assert np.array_equal(list0, both["list0"]) and np.array_equal(lst[:int(list0[-1])], both["list"])
 
 
+@pytest.mark.parametrize("seed", [0, 5, 161])
+def test_final_lists_without_room(oracle, ctx, tmp_path, seed):
+    """the final lists made on the host where the device has no room for their
+    scratch; the last level of seed 161 got its refinement's particles back"""
+    snap = str(tmp_path / "rb.snap")
+    fuzz_snapshot(snap, seed)
+    assert oracle.oracle_amr_dump(snap.encode(), str(tmp_path / "o.grid").encode()) > 0
+    info = _gpu_dump(ctx, snap, str(tmp_path / "g.grid"))
+    assert (info.rolled_back == 1) == (seed == 161)
+    with_room = [ctx.amr_level(lev) for lev in range(info.n_levels)]
+    try:
+        ctx.set_memory_limit(1)
+        ctx.amr_dump(str(tmp_path / "h.grid"))
+        without = [ctx.amr_level(lev) for lev in range(info.n_levels)]
+    finally:
+        ctx.set_memory_limit(0)
+    assert not dumps.compare_grids(dumps.read_grids(str(tmp_path / "h.grid")), dumps.read_grids(str(tmp_path / "o.grid")))
+    for a, b in zip(with_room, without):
+        assert np.array_equal(a["list0"], b["list0"]) and np.array_equal(a["list"], b["list"])
+
+
 @pytest.mark.parametrize("n", [32, 33, 1024, 1025, 4096, 4097, 8193, 30000])
 def test_fine_buckets(oracle, ctx, tmp_path, n):
     """a node's bucket at the edges of the three ways to split it among the

@@ -269,7 +269,8 @@ def _form_snapshot(path, seed):
                                                     (0, -1, 0.0, dict(big_halo=600, wave_halo=70)), (0, 300, 0.0, {})])
 def test_form_sizes(oracle, ctx, tmp_path, cuts, plain, split, band, sched):
     """haloes on both sides of every size at which the unbinding changes its
-    form, in every form that can hold them, some sent to the exact replay"""
+    form, in the forms that a few haloes take (test_many_short_haloes has the
+    others), some sent to the exact replay"""
     snap, out = str(tmp_path / "f.snap"), str(tmp_path / "o.halo")
     _form_snapshot(snap, 5)
     dump = oracle.oracle_construct_dump if cuts else oracle.oracle_unbind_dump
@@ -454,6 +455,22 @@ def test_rounding_edge(oracle, ctx, tmp_path, split):
     info, (npart, props, lists) = _run_gpu(ctx, dumps.read_snapshot(snap), 0, split=split)
     assert info.n_exact_replays >= 12
     _compare(ref, npart, props, lists, f"edge split {split}")
+
+
+@pytest.mark.parametrize("cuts", [0, WITH_RVIR])
+def test_many_short_haloes(oracle, ctx, tmp_path, cuts):
+    """more short haloes than are resident at once: the one-wavefront forms in
+    launches of their own, from the host's order and from the cut's lists"""
+    from helpers import short_haloes_snapshot
+    snap, out = str(tmp_path / "s.snap"), str(tmp_path / "o.halo")
+    left = short_haloes_snapshot(snap, 6, 5000)
+    assert all(np.count_nonzero(x) > 20 for x in (left < 128, (left > 128) & (left < 512), left > 512))
+    dump = oracle.oracle_construct_dump if cuts else oracle.oracle_unbind_dump
+    assert dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    s = dumps.read_snapshot(snap)
+    _, (npart, props, lists) = _construct_gpu(ctx, s, cuts) if cuts else _run_gpu(ctx, s, 0)
+    _compare(ref, npart, props, lists, f"short haloes {cuts}")
 
 
 def test_schedule_file(tmp_path, monkeypatch):

@@ -147,6 +147,23 @@ def test_noalloc_matches_unbind(snapgen, ctx, tmp_path, cfg, side, seed, mode):
         hip.close()
 
 
+@pytest.mark.parametrize("mode", [0, 16])
+def test_noalloc_many_short_haloes(ctx, tmp_path, mode):
+    """more haloes than one launch takes for both one-wavefront forms, against
+    the form that unbinds one halo a launch"""
+    from helpers import short_haloes_snapshot
+    snap = str(tmp_path / "s.snap")
+    short_haloes_snapshot(snap, 7, 5000)
+    s = dumps.read_snapshot(snap)
+    ctx.set_particles(s.pos, s.mom)
+    hip = Hip()
+    try:
+        ref = _existing(ctx, s, s.nhalos, mode | 1)
+        _same(ref, _noalloc(ctx, hip, s, s.nhalos, mode), f"short haloes mode {mode}")
+    finally:
+        hip.close()
+
+
 def test_noalloc_rejects_too_many_haloes(ctx):
     import ahf_amd
     lib = ctx.lib
