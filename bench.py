@@ -171,17 +171,24 @@ def copy_probe(nbytes=1 << 30, reps=5):
         hip.hipFree(b)
 
 
-def load_traffic():
+# the kernels of the deposit's timed launches: on levels holding every octet,
+# and on the others
+DEPOSIT_KERNELS = ("k_gather_full", "k_gather_light")
+
+
+def load_traffic(workload, path=os.path.join(ROOT, "profiles", "deposit_traffic.json")):
     """HBM bytes per deposit launch (one grid level) of this workload,
     measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE over the deposit
     kernels and scaled by the copy-kernel calibration
     (profiles/deposit_traffic.json, written by
-    python -m ahf_amd.rocprof_summary traffic)."""
-    path = os.path.join(ROOT, "profiles", "deposit_traffic.json")
+    python -m ahf_amd.rocprof_summary traffic); None when the file is of
+    another workload or of other kernels than the timed ones."""
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        return json.load(f)
+        t = json.load(f)
+    kernels = {k.replace("void ", "").split("<")[0].strip() for k in t.get("kernel", "").split(" + ")}
+    return t if t.get("workload") == workload and kernels == set(DEPOSIT_KERNELS) else None
 
 
 def unbinding_workload(seed=1002, reps=3, cpu=True, threads=16):
@@ -441,10 +448,7 @@ def main():
     # wavefront-per-node folds of the heaviest nodes (gather_heavy)
     dep_ms = stage_ms["prep"] + stage_ms["gather_light"] + stage_ms["gather_heavy"]
     achieved_incl = dep_bytes / (dep_ms * 1e-3) / 1e9
-    traffic = load_traffic()
-    cfg_tag = f"cfg{args.config}_{args.side}_{args.seed}"
-    if traffic and traffic.get("workload") != cfg_tag:
-        traffic = None
+    traffic = load_traffic(f"cfg{args.config}_{args.side}_{args.seed}")
 
     out = {
         "metric": METRIC,
@@ -483,8 +487,8 @@ def main():
         "stage_ms": stage_ms,
         "dominant_stage": dom,
         "roofline": {
-            "kernel": ("exact-order TSC deposit, one timed launch per grid level: k_gather_full "
-                       "on levels holding every octet, k_gather_light on the others"),
+            "kernel": ("exact-order TSC deposit, one timed launch per grid level: %s "
+                       "on levels holding every octet, %s on the others") % DEPOSIT_KERNELS,
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
