@@ -7,8 +7,12 @@
  * resident in HBM.  Per level the kernels are:
  *
  *   k_pmask        presence mask of every node (get_TSCnodes rules)
- *   k_prep         particle-node separations of every bucket entry
- *   k_gather_light exact-order TSC density, one lane per node (assign_npart)
+ *   k_prep         TSC weights and position of every bucket entry (k_prep_q:
+ *                  the position alone, on levels that march or walk per source)
+ *   k_gather_full  exact-order TSC density (assign_npart) of a level that holds
+ *                  every octet, marching through its planes
+ *   k_gather_light the same on the others, one lane per node (k_gather_src:
+ *                  many entries per node)
  *   k_gather_heavy the same, nodes with many contributions, by wavefronts
  *   k_flags        interior + refinement criterion (test_node)
  *   k_refine_rows  ref_pquad/ref_cquad/ref_nquad block tests and run state
@@ -2276,11 +2280,13 @@ static int64_t march_planes(int64_t L, int64_t side)
 }
 
 /*
- * Exact-order gather of one level over its n_ent bucket entries: the octets
- * sorted into Morton order (the target order), then either
- *  - dense levels (many entries per node): a position record per entry and
- *    the per-source walk (k_gather_src), whose records stay in L2; or
- *  - sparse levels: a TSC weight record per entry and the flat walk
+ * Exact-order gather of one level over its n_ent bucket entries, a position
+ * record each: levels that hold every octet and are not small march
+ * (k_gather_full); on the others the octets are sorted into Morton order (the
+ * target order), and then either
+ *  - dense levels (many entries per node): the per-source walk
+ *    (k_gather_src), whose records stay in L2; or
+ *  - sparse levels: a TSC weight record per entry as well and the flat walk
  *    (k_gather_light), which keeps a wavefront's lanes busy when buckets
  *    hold a particle or two;
  * and by wavefronts the nodes with more than kmax contributions.  Every

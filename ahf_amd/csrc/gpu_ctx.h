@@ -104,7 +104,7 @@ struct DevLevel {
   uint32_t *plist = nullptr;
   uint32_t *pnode = nullptr;   /* per bucket entry: its node */
   ahf_w9 *W = nullptr;                              /* per bucket entry: TSC weights (sparse)     */
-  ahf_q4 *qp = nullptr;                             /* per bucket entry: position (dense levels)  */
+  ahf_q4 *qp = nullptr;                             /* per bucket entry: position                 */
   uint32_t *tord = nullptr;                         /* octets in Morton order                      */
   int8_t *child = nullptr;     /* per bucket entry: fine child it moved to, or -1 */
   int32_t *node2oct = nullptr; /* per node: octet of the next level, or -1 */
@@ -140,14 +140,14 @@ struct ahfgpu_ctx {
   int device = 0;
   hipStream_t st = nullptr;
   hipStream_t st2 = nullptr; /* the split unbinding path beside st (default priority) */
-  hipStream_t st3 = nullptr; /* the one-wavefront unbinding tier beside st (default priority) */
+  hipStream_t st3 = nullptr; /* the one-wavefront unbinding forms beside st (default priority) */
   hipEvent_t ev_s0 = nullptr, ev_s1 = nullptr, ev_s2 = nullptr, ev_s3 = nullptr;
   int64_t split_min = 0;     /* haloes of at least this many members take the split path; 0: default */
   int64_t prof_split = 0;    /* haloes of at least this many members are profiled by four wavefronts; 0: default */
   /* the rest of the schedule (ahfgpu_schedule); 0: the default */
-  int32_t kmax_big = 0, kmax_small = 0; /* contributions above which a node's density is folded by a wavefront */
+  int32_t kmax_big = 0, kmax_small = 0; /* contributions above which a node's density is folded by wavefronts */
   int32_t march_zn = 0;                 /* target planes per march workgroup */
-  int64_t big_halo = 0, wave_halo = 0;  /* unbinding tiers: 512-thread workgroups from, one wavefront below */
+  int64_t big_halo = 0, wave_halo = 0;  /* unbinding: 512-thread workgroups from, one wavefront below */
   char err[512] = {0};
   Arena arena;        /* AMR build buffers */
   Arena uarena;       /* unbinding buffers */

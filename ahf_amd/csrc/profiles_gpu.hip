@@ -506,12 +506,15 @@ __device__ void prf_radii(const ProfConst &K, int64_t n, const uint32_t *__restr
  * that decrease keep the sequential walk.
  */
 #define PRF_TILE 1024
-/* the default prof_tiled.  A member costs a lane's chain of additions some 10
- * ns there, k_profiles<4> some 30 ns (one workgroup's barriers), and the
- * longest walk is what the call waits for: from 32768 on instead of 8192, the
- * profiles of a 128^3 catalogue took 1.1 to 1.2 ms for 0.72 to 0.90, of a
- * 256^3 one with haloes of 8000 0.67 for 0.43, of 20,000 haloes 1.38 for 0.76
- * where none was larger; from 4096 on nothing more.  The rows take 164 bytes a
+/* the default prof_tiled.  k_prf_walk takes 5 to 6 ns a member (260,921 members
+ * 1.33 ms, 1,350,831 7.96), k_profiles<4> 33 to 38 (one workgroup's barriers),
+ * and the longest walk is what the call waits for.  Profiles alone, from 32768
+ * on and from 8192 on, the same haloes: 128^3 catalogues 1.21 and 0.91 ms, 1.08
+ * and 0.72 (two others, whose largest halo sets the time either way, the
+ * same); 256^3 ones with a largest halo of 16,676 0.74 and 0.47, of 15,072 0.67
+ * and 0.42; 20,000 haloes with a largest of 49,417 1.40 and 0.76, with larger
+ * ones the same.  From 4096 on the two 256^3 ones took 0.31 and 0.32, the others
+ * what they take from 8192 on.  The rows take 164 bytes a
  * member: haloes below AHF_PROF_TILED_ANY only while all of them together have
  * at most AHF_PROF_TILED_SUM, and only where the device has room for the rows. */
 #define AHF_PROF_TILED 8192

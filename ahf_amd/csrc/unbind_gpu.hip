@@ -9,9 +9,10 @@
  *    input order.  Haloes below NminPerHalo keep their order (AHF does not
  *    sort them).
  * 2. Unbinding: persistent kernels by size, a wavefront or a workgroup per
- *    halo that keeps the halo's members in registers, haloes taken largest
- *    first from an atomic queue; the largest haloes over the chip (the split
- *    path).  Per iteration:
+ *    halo that keeps the halo's members in registers, haloes taken from an
+ *    atomic queue: largest first in the host's order, in no order within a
+ *    form where the lists are made on the device (k_bin_forms); the largest
+ *    haloes over the chip (the split path).  Per iteration:
  *      - dist_j, the mid-point terms of the integral of M(<r)/r^2 and their
  *        FP64 prefix sum Phi_j; Phi0 = Phi_{n-1} + n/dist_{n-1} (AHF's two
  *        passes add the same terms in the same order);
@@ -25,9 +26,9 @@
  *        the escape test this bounds, per member, how far the sequential
  *        vel^2 and limit can lie from the parallel ones.  A member whose
  *        margin is inside that bound (or inside `band`, relative, if the
- *        caller asks for more) sends the halo to an exact sequential replay
- *        of the iteration in AHF's own operation order; every other
- *        decision is the sequential one;
+ *        caller asks for more) sends the iteration to exact_iteration, which
+ *        decides it from running sums in AHF's own operation order; every
+ *        other decision is the sequential one;
  *      - stable compaction of the bound members.
  * 3. rem_outsideRvir (:3687-3889), on request before and after the
  *    unbinding as ahf_halos_sfc.c:143,153 call it: the overdensity of the
@@ -1690,9 +1691,10 @@ static inline unsigned seed_blocks(int64_t nh)
  * wave_halo move the lines between the register forms below that.  The
  * kernels are bound by the serial chain of the longest halo's iterations, not
  * by memory: in registers an iteration has no pass over memory and one barrier
- * a hand-over.  Against chunks for every size (unbinding alone): 2,000 lists of
- * 20 to 100,000 members 0.82 -> 0.77 ms, 20,000 lists 1.74 -> 1.39 ms, and 16
- * lists end to end 213 -> 192 us.
+ * a hand-over.  Against chunks for every size, whole calls on the same lists:
+ * 4,000 lists in the caller's memory 3.02 -> 2.20 ms (5.63 -> 5.42 with others,
+ * whose largest is longer), 2,000 lists 1.29 -> 1.20, 20,000 with a largest of
+ * more than 10^6 11.06 -> 10.61, 16 lists the same within the spread.
  */
 enum { UF_CHUNK = 0, UF_BIG, UF_MID, UF_WAVE, UF_SMALL, UF_FORMS };
 #define AHF_BIG_BLOCK 512
@@ -1723,8 +1725,8 @@ static inline bool uf_either(bool binned, int64_t haloes, int cu) { return haloe
  * 8 members and an evaluation's temporaries, 128 hold 2 */
 #define AHF_UNBIND_WAVES(IPT) ((IPT) == 2 ? 4 : 2)
 
-/* persistent form: workgroups take haloes order[q0..q1) from the queue
- * (largest first) */
+/* persistent form: workgroups take haloes order[q0..q1) from the queue, in
+ * order's order */
 template <int BS, int IPT>
 __device__ __forceinline__ void unbind_queue(const UnbindConst &K, const int64_t *__restrict__ off,
                                              const int32_t *__restrict__ order, int64_t q0, int64_t q1,
@@ -1830,8 +1832,9 @@ __device__ __forceinline__ int64_t group_cut(const UnbindConst &K, int64_t n, co
  * twenty): in the form of its full list the cut members would be carried
  * through every iteration.  A halo that is chunked at any rate makes its cut
  * there (pad: the cut is still to be made).  The record's fields are the
- * cut's, or cleared.  (2.8 million gathered members, 2,400 haloes: 15 us; cut
- * 1,024 members a step 50 us, for the records beyond the cut.)
+ * cut's, or cleared.  Every form waits for it: 43 us for the 2,437 gathered
+ * haloes of a 256^3 box, 57 for 4,000 lists, 238 for 20,000 (random reads of
+ * records, most of them beyond the cut: so the step of 256 members first).
  */
 __global__ void __launch_bounds__(AHF_BLOCK) k_bin_forms(UnbindConst K, const int64_t *__restrict__ off,
                                                   const int32_t *__restrict__ order, int64_t q0, int64_t nh,
@@ -3318,9 +3321,9 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
   } else if (run == 0) {
     /* the order is largest first: haloes of split_min members or more take
      * the split path on the second stream, the others the forms by size: the
-     * wavefront forms on the third stream, the workgroup forms on the first,
-     * the chunked one (only with split_min above its size) behind the split
-     * path's start */
+     * wavefront forms on the third stream, the workgroup forms on the first
+     * (which stream the chunked form, 4097 members to split_min, has depends on
+     * the split path: below) */
     int64_t nsplit = 0;
     const std::vector<int32_t> &ord = s->h_ord;
     const int64_t split_min = c->split_min > 0 ? c->split_min : AHF_SPLIT_DEFAULT;
@@ -3345,8 +3348,8 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     int32_t *list = nullptr, *cnt = next + UF_FORMS;
     const bool either = uf_either(binned, binned ? nh - nsplit : q0[UF_FORMS] - q0[UF_WAVE], dev_cu);
     if (either) least.v[UF_WAVE] = 0;
-    /* the split path is used where one halo needs it (below); its haloes take
-     * the cut there */
+    /* the most haloes that form f can get (the split path's take their cut
+     * there) */
     auto most = [&](int f) { return binned ? q0[f + 1] - nsplit : q0[f + 1] - q0[f]; };
     if (binned) {
       list = A.get<int32_t>(UF_FORMS * nh);

@@ -314,10 +314,13 @@ int ahfgpu_gridinfo_results(ahfgpu_ctx *ctx, int grid, int32_t *colour, int32_t 
 typedef struct {
   int64_t split_min;   /* haloes of this many members or more take the split path (-1: none); 16384 */
   int64_t prof_split;  /* HaloProfiles: haloes of this many members or more on four wavefronts (-1: none); 2048 */
-  int64_t big_halo;    /* unbinding: haloes of this many members or more on 512-thread workgroups; 2049 (at most) */
-  int64_t wave_halo;   /* unbinding: haloes below this many members on one wavefront; 513 (at most) */
+  int64_t big_halo;    /* unbinding: haloes of this many members or more on 512-thread workgroups; 2049, and larger
+                          values act as 2049 (what 256 threads hold in registers) */
+  int64_t wave_halo;   /* unbinding: haloes below this many members on one wavefront; 513, and larger values act as
+                          513 (what a wavefront holds in registers) */
   int32_t kmax_big;    /* deposit: nodes with more contributions folded by wavefronts (levels of 2^21 nodes or more);
-                          1.5 times the level's mean, at least 96 */
+                          on levels that march (every octet there, 40 nodes a side or more) 1.5 times the level's
+                          mean, within [96, 2000], on the others 96 */
   int32_t kmax_small;  /* ... on smaller levels; the same */
   int32_t march_zn;    /* deposit: target planes per march workgroup (8 or 16); by level size */
   int32_t graph_batch; /* split unbinding: iteration graph replays between done checks; 4 */

@@ -1,6 +1,6 @@
 /*
  * march_rows_check.c -- host check of the march kernel's rows walk
- * (ahf_amd/csrc/amr_gpu.hip, k_gather_march, the rows fast path): for
+ * (ahf_amd/csrc/amr_gpu.hip, gather_march, the rows fast path): for
  * random entry counts of a staged 18x18 source plane and lanes inside the
  * box and at the periodic faces, the entries the walk visits with the
  * functions it uses (ahf_row_start / ahf_row_next / ahf_row_src) must be
