@@ -2149,8 +2149,15 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
       hipEventRecord(c->ev_s1, c->st2);
     }
     /* the small haloes: behind the peaks on the third stream where the first
-     * has big ones to walk */
-    hipStream_t s1 = ntl && nbig > ntl ? c->st3 : c->st;
+     * has big ones to walk (20,000 haloes with a largest of 49,417 0.99 -> 0.74
+     * ms).  k_prf_walk takes all of a CU's LDS: where the big haloes' workgroups
+     * occupy every CU, it starts when they leave, unless small ones took their
+     * places at once (100,000 haloes, 699 big ones on workgroups: 4.53 ms, or up
+     * to 7.04 with the small ones on the third stream).  So only while the big
+     * haloes leave CUs free. */
+    int dev_cu = 256;
+    hipDeviceGetAttribute(&dev_cu, hipDeviceAttributeMultiprocessorCount, c->device);
+    hipStream_t s1 = ntl && nbig > ntl && nbig <= dev_cu ? c->st3 : c->st;
     hipLaunchKernelGGL(k_profiles<1>, dim3((unsigned)nh), dim3(64), 0, s1, K, s->off, s->order, big, out, d_pr,
                        s->ip_in, s->buf_a, s->buf_b, s->cen, d_nb, d_pofs, c->px, c->py, c->pz, c->vx, c->vy, c->vz,
                        sc, sc + ne, sc + 2 * ne, r->props, r->prof, (const PrfTiled *)nullptr,

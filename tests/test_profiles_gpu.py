@@ -154,6 +154,23 @@ def test_profiles_walk_line(ctx, sizes):
     _same_profiles(*got)
 
 
+@pytest.mark.parametrize("sizes", [(8192,) + 255 * (2050,) + (300,),
+                                   (8192,) + 256 * (2050,) + (300,)])
+def test_profiles_beside_others(ctx, sizes):
+    """as many big haloes as there are CUs, and one more, give the bits of the
+    walk on one workgroup"""
+    centre, ip, pr = _given_haloes(ctx, sizes)
+    got = []
+    try:
+        for tiled in (0, -1):
+            ctx.set_schedule(prof_tiled=tiled)
+            ctx.set_halos(centre, np.array(sizes, np.int64), ip)
+            got.append(ctx.halo_profiles(20, 1.0, 1.0, 1.0, 1.0, 0.1, phi0_rvir=pr))
+    finally:
+        _reset_split(ctx)
+    _same_profiles(*got)
+
+
 @pytest.mark.parametrize("sizes,fits", [((32767, 8192, 300), 0), ((40000, 32767, 8192, 300), 40000), ((40000, 300), None)])
 def test_profiles_without_room(ctx, sizes, fits):
     """haloes below 32768 members do without the rows of the walk over the
