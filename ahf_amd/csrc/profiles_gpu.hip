@@ -514,11 +514,18 @@ __device__ void prf_radii(const ProfConst &K, int64_t n, const uint32_t *__restr
  * same); 256^3 ones with a largest halo of 16,676 0.74 and 0.47, of 15,072 0.67
  * and 0.42; 20,000 haloes with a largest of 49,417 1.40 and 0.76, with larger
  * ones the same.  From 4096 on the two 256^3 ones took 0.31 and 0.32, the others
- * what they take from 8192 on.  The rows take 164 bytes a
+ * what they take from 8192 on.  Beside a much larger halo, whose walk covers
+ * the smaller ones' on one workgroup, their passes ahead of the walk only delay
+ * it: haloes below AHF_PROF_TILED_ANY are walked over the device from a part of
+ * 1/AHF_PROF_TILED_PART of the largest on (100,000 haloes, the largest of
+ * 809,536, with all from 8192 on 4.79 ms, with a part of 1/8 4.53; 128^3
+ * catalogues gain to the full down to 1/8, at 1/6 they lose up to 0.36 ms of
+ * 0.91).  The rows take 164 bytes a
  * member: haloes below AHF_PROF_TILED_ANY only while all of them together have
  * at most AHF_PROF_TILED_SUM, and only where the device has room for the rows. */
 #define AHF_PROF_TILED 8192
 #define AHF_PROF_TILED_ANY 32768
+#define AHF_PROF_TILED_PART 8
 #define AHF_PROF_TILED_SUM ((int64_t)1 << 25)
 
 struct PrfTiled {
@@ -2010,7 +2017,10 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
     for (int32_t h : bigl) {
       const int64_t n = hn[(size_t)h];
       /* largest first: the haloes walked over the device are the list's first */
-      if (n < least || (c->prof_tiled == 0 && n < AHF_PROF_TILED_ANY && Nt + n > AHF_PROF_TILED_SUM)) break;
+      if (n < least) break;
+      if (c->prof_tiled == 0 && n < AHF_PROF_TILED_ANY &&
+          (Nt + n > AHF_PROF_TILED_SUM || n * AHF_PROF_TILED_PART < hn[(size_t)bigl[0]]))
+        break;
       if (tmap_h.empty()) tmap_h.assign((size_t)nh, -1);
       PrfTiled T;
       memset(&T, 0, sizeof(T));

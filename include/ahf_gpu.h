@@ -328,7 +328,8 @@ typedef struct {
                           resumes (-1: none); 3 */
   int32_t pad;
   int64_t prof_tiled;  /* HaloProfiles: haloes of this many members or more walked by kernels over the
-                          whole device, only their running sums sequential (-1: none); 8192 */
+                          whole device, only their running sums sequential (-1: none); 8192, or below 32768 an
+                          eighth of the largest halo's members, if more */
 } ahfgpu_schedule;
 int ahfgpu_set_schedule(ahfgpu_ctx *ctx, const ahfgpu_schedule *s);
 int ahfgpu_get_schedule(ahfgpu_ctx *ctx, ahfgpu_schedule *s);

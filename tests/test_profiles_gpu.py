@@ -154,11 +154,12 @@ def test_profiles_walk_line(ctx, sizes):
     _same_profiles(*got)
 
 
-@pytest.mark.parametrize("sizes", [(8192,) + 255 * (2050,) + (300,),
+@pytest.mark.parametrize("sizes", [(70000, 8750, 8749, 2500, 300), (8192,) + 255 * (2050,) + (300,),
                                    (8192,) + 256 * (2050,) + (300,)])
 def test_profiles_beside_others(ctx, sizes):
-    """as many big haloes as there are CUs, and one more, give the bits of the
-    walk on one workgroup"""
+    """haloes on both sides of the part of the largest from which they are
+    walked over the device beside it, and as many big ones as there are CUs and
+    one more, give the bits of the walk on one workgroup"""
     centre, ip, pr = _given_haloes(ctx, sizes)
     got = []
     try:
