@@ -3414,15 +3414,26 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     }
   } else {
     /* plain form: one halo per launch, results synchronised per halo as a
-     * per-call rem_unbound() would need them */
+     * per-call rem_unbound() would need them.  The forms of the batched call by
+     * size, and the record alone below NminPerHalo: the register form's 256
+     * threads take 5 us for a list of nothing.  The 2,437 lists of a 256^3 box
+     * (2,151 of them below NminPerHalo) 31.9 ms, with 256 threads for all up to
+     * 2048 members 49.5, in chunks 36.1; 2,000 of 20 to 36,735 members 51, 95
+     * and 76. */
+    int64_t least[UF_FORMS];
+    for (int f = 0; f < UF_FORMS; f++) least[f] = uf_least(c, f);
     for (int64_t h = 0; h < nh; h++) {
       const int64_t n = s->h_off[h + 1] - s->h_off[h];
 #define AHF_UNBIND_ONE(BS, IPT)                                                                                   \
   hipLaunchKernelGGL((k_unbind_one<BS, IPT>), dim3(1), dim3(BS), 0, c->st, K, h, s->off, seed, s->buf_a, s->buf_b, \
                      dist, phi, st, g, s->cen, c->pv, s->out)
-      if (n > AHF_BIG_MOST) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 0);
-      else if (n >= uf_least(c, UF_BIG)) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 8);
-      else AHF_UNBIND_ONE(AHF_BLOCK, 8);
+      if (n < p->minpart)
+        hipLaunchKernelGGL(k_sorted_out, dim3(1), dim3(64), 0, c->st, s->off + h, (int64_t)1, s->out + h);
+      else if (n >= least[UF_CHUNK]) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 0);
+      else if (n >= least[UF_BIG]) AHF_UNBIND_ONE(AHF_BIG_BLOCK, 8);
+      else if (n >= least[UF_MID]) AHF_UNBIND_ONE(AHF_BLOCK, 8);
+      else if (n >= least[UF_WAVE]) AHF_UNBIND_ONE(64, 8);
+      else AHF_UNBIND_ONE(64, 2);
 #undef AHF_UNBIND_ONE
       hipStreamSynchronize(c->st);
     }
