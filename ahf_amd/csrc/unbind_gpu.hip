@@ -3343,6 +3343,9 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
      * size or more */
     const bool binned = K.cut_before != 0 && nh > nsplit;
     UnbindConst KF = K;
+    /* k_bin_forms makes the whole record where the cut is all there is to do:
+     * only the chunked form, which makes its own, runs behind it */
+    const bool cut_only = binned && !K.unbind;
     FormLeast least;
     for (int f = 0; f < UF_FORMS; f++) least.v[f] = uf_least(c, f);
     int32_t *list = nullptr, *cnt = next + UF_FORMS;
@@ -3350,7 +3353,9 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     if (either) least.v[UF_WAVE] = 0;
     /* the most haloes that form f can get (the split path's take their cut
      * there) */
-    auto most = [&](int f) { return binned ? q0[f + 1] - nsplit : q0[f + 1] - q0[f]; };
+    auto most = [&](int f) {
+      return cut_only && f != UF_CHUNK ? 0 : binned ? q0[f + 1] - nsplit : q0[f + 1] - q0[f];
+    };
     if (binned) {
       list = A.get<int32_t>(UF_FORMS * nh);
       if (!list) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (unbinding)");
@@ -3360,8 +3365,8 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     }
     /* the other streams start after the sort, the seeds and the queue
      * counters; with a single form and no split path there is no hand-over */
-    const int64_t wgs = q0[UF_WAVE] - nsplit, wvs = binned ? nh - nsplit : q0[UF_FORMS] - q0[UF_WAVE];
-    const bool fork = nsplit > 0 || (wgs > 0 && wvs > 0) || (q0[UF_BIG] > nsplit && nh > q0[UF_BIG]);
+    const int64_t wgs = q0[UF_WAVE] - nsplit, wvs = cut_only ? 0 : binned ? nh - nsplit : q0[UF_FORMS] - q0[UF_WAVE];
+    const bool fork = nsplit > 0 || (!cut_only && ((wgs > 0 && wvs > 0) || (q0[UF_BIG] > nsplit && nh > q0[UF_BIG])));
     if (fork) hipEventRecord(c->ev_s0, c->st);
     /* F: the form's counters; Q: its first halo in the host's order */
 #define AHF_UNBIND_LAUNCH(F, Q, N, BS, IPT, PER_CU, STREAM)                                                              \
@@ -3825,6 +3830,8 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
                        (const int32_t *)nullptr, (int64_t)0, nh, least, buf_a, centres, c->pv, list, cnt, hout);
     UnbindConst KF = K;
     if (K.cut_before) KF.cut_before = CUT_DONE;
+    /* the cut alone: as in the batched form */
+    const bool cut_only = K.cut_before && !K.unbind;
     hipEventRecord(c->ev_s0, st);
     hipStreamWaitEvent(c->st2, c->ev_s0, 0);
     hipStreamWaitEvent(c->st3, c->ev_s0, 0);
@@ -3833,14 +3840,18 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
                      dim3(BS), 0, STREAM, KF, off, list + (F) * nh, cnt + (F), next + (F), seed, buf_a, buf_b,    \
                      dist, phi, stt, g, centres, c->pv, hout);
     AHF_UNBIND_LAUNCH(UF_CHUNK, AHF_BIG_BLOCK, 0, 2, c->st2)
-    if (either) {
+    if (cut_only) {
+      /* the records are made */
+    } else if (either) {
       AHF_UNBIND_LAUNCH(UF_WAVE, 64, UF_EITHER, 8, c->st3)
     } else {
       AHF_UNBIND_LAUNCH(UF_WAVE, 64, 8, 8, c->st3)
       AHF_UNBIND_LAUNCH(UF_SMALL, 64, 2, 16, c->st3)
     }
-    AHF_UNBIND_LAUNCH(UF_BIG, AHF_BIG_BLOCK, 8, 1, st)
-    AHF_UNBIND_LAUNCH(UF_MID, AHF_BLOCK, 8, 2, st)
+    if (!cut_only) {
+      AHF_UNBIND_LAUNCH(UF_BIG, AHF_BIG_BLOCK, 8, 1, st)
+      AHF_UNBIND_LAUNCH(UF_MID, AHF_BLOCK, 8, 2, st)
+    }
 #undef AHF_UNBIND_LAUNCH
     hipEventRecord(c->ev_s1, c->st2);
     hipEventRecord(c->ev_s2, c->st3);

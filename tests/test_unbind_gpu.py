@@ -297,6 +297,32 @@ def test_form_sizes(oracle, ctx, tmp_path, cuts, plain, split, band, sched):
         assert np.array_equal(ref.ovdens, props[:, 3])
 
 
+@pytest.mark.parametrize("split", [0, -1])
+def test_rvir_only_form_sizes(ctx, tmp_path, split):
+    """the cut alone, batched and in the call that allocates nothing, gives the
+    records and lists of one halo a launch, on both sides of every form's line"""
+    from test_zz_no_alloc import Hip, _noalloc
+    snap = str(tmp_path / "f.snap")
+    _form_snapshot(snap, 9)
+    s = dumps.read_snapshot(snap)
+    off, ip = s.halo_offsets, s.ipart.copy()
+    for h in range(s.nhalos):
+        seg = ip[off[h]:off[h + 1]].astype(np.int64)
+        d = np.abs(s.pos[seg].astype(np.float64) - s.centre[h])
+        ip[off[h]:off[h + 1]] = seg[np.argsort((np.minimum(d, 1.0 - d) ** 2).sum(1))]
+    s.ipart = ip
+    _, (np0, pr0, li0) = _construct_gpu(ctx, s, 1 | RVIR_ONLY, ipart=ip)
+    assert np.sum(np0 < s.halo_npart) > 5 and pr0[:, 0].max() > 0
+    hip = Hip()
+    try:
+        for got in (_construct_gpu(ctx, s, RVIR_ONLY, ipart=ip, split=split)[1], _noalloc(ctx, hip, s, s.nhalos, RVIR_ONLY)):
+            assert np.array_equal(np0, got[0]) and np.array_equal(pr0, got[1])
+            assert all(np.array_equal(a, b) for a, b in zip(li0, got[2]))
+    finally:
+        hip.close()
+        ctx.set_unbind_split(0)
+
+
 ODD = [(n, where, value) for n in (300, 600, 2000, 4000, 5000) for where in ("first", "middle", "last")
        for value in ("nan", "inf", "both")]
 
