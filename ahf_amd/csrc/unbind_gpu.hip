@@ -3820,7 +3820,9 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
     int dev_cu = 256;
     hipDeviceGetAttribute(&dev_cu, hipDeviceAttributeMultiprocessorCount, c->device);
     /* the forms on the three streams, as in the batched form, over lists made
-     * on the device (with the cut ahead of the unbinding, if any) */
+     * on the device (with the cut ahead of the unbinding, if any).  The sizes
+     * are on the device, their sum here: forms that no list can need are not
+     * launched. */
     FormLeast least;
     for (int f = 0; f < UF_FORMS; f++) least.v[f] = uf_least(c, f);
     const bool either = uf_either(true, nh, dev_cu);
@@ -3832,31 +3834,38 @@ extern "C" int ahfgpu_unbind_noalloc(ahfgpu_ctx *c, const ahfgpu_unbind_params *
     if (K.cut_before) KF.cut_before = CUT_DONE;
     /* the cut alone: as in the batched form */
     const bool cut_only = K.cut_before && !K.unbind;
-    hipEventRecord(c->ev_s0, st);
-    hipStreamWaitEvent(c->st2, c->ev_s0, 0);
-    hipStreamWaitEvent(c->st3, c->ev_s0, 0);
+    const bool chunk = ne >= least.v[UF_CHUNK], big = !cut_only && ne >= least.v[UF_BIG],
+               mid = !cut_only && ne >= least.v[UF_MID], fork = big || mid || (chunk && !cut_only);
+    hipStream_t sc = fork ? c->st2 : st, sw = fork ? c->st3 : st;
+    if (fork) {
+      hipEventRecord(c->ev_s0, st);
+      if (chunk) hipStreamWaitEvent(sc, c->ev_s0, 0);
+      hipStreamWaitEvent(sw, c->ev_s0, 0);
+    }
 #define AHF_UNBIND_LAUNCH(F, BS, IPT, PER_CU, STREAM)                                                             \
   hipLaunchKernelGGL((k_unbind_dq<BS, IPT>), dim3((unsigned)std::min<int64_t>(nh, (int64_t)dev_cu * (PER_CU))),   \
                      dim3(BS), 0, STREAM, KF, off, list + (F) * nh, cnt + (F), next + (F), seed, buf_a, buf_b,    \
                      dist, phi, stt, g, centres, c->pv, hout);
-    AHF_UNBIND_LAUNCH(UF_CHUNK, AHF_BIG_BLOCK, 0, 2, c->st2)
+    if (chunk) AHF_UNBIND_LAUNCH(UF_CHUNK, AHF_BIG_BLOCK, 0, 2, sc)
     if (cut_only) {
       /* the records are made */
     } else if (either) {
-      AHF_UNBIND_LAUNCH(UF_WAVE, 64, UF_EITHER, 8, c->st3)
+      AHF_UNBIND_LAUNCH(UF_WAVE, 64, UF_EITHER, 8, sw)
     } else {
-      AHF_UNBIND_LAUNCH(UF_WAVE, 64, 8, 8, c->st3)
-      AHF_UNBIND_LAUNCH(UF_SMALL, 64, 2, 16, c->st3)
+      AHF_UNBIND_LAUNCH(UF_WAVE, 64, 8, 8, sw)
+      AHF_UNBIND_LAUNCH(UF_SMALL, 64, 2, 16, sw)
     }
-    if (!cut_only) {
-      AHF_UNBIND_LAUNCH(UF_BIG, AHF_BIG_BLOCK, 8, 1, st)
-      AHF_UNBIND_LAUNCH(UF_MID, AHF_BLOCK, 8, 2, st)
-    }
+    if (big) AHF_UNBIND_LAUNCH(UF_BIG, AHF_BIG_BLOCK, 8, 1, st)
+    if (mid) AHF_UNBIND_LAUNCH(UF_MID, AHF_BLOCK, 8, 2, st)
 #undef AHF_UNBIND_LAUNCH
-    hipEventRecord(c->ev_s1, c->st2);
-    hipEventRecord(c->ev_s2, c->st3);
-    hipStreamWaitEvent(st, c->ev_s1, 0);
-    hipStreamWaitEvent(st, c->ev_s2, 0);
+    if (fork) {
+      if (chunk) {
+        hipEventRecord(c->ev_s1, sc);
+        hipStreamWaitEvent(st, c->ev_s1, 0);
+      }
+      hipEventRecord(c->ev_s2, sw);
+      hipStreamWaitEvent(st, c->ev_s2, 0);
+    }
   }
   hipLaunchKernelGGL(k_na_out_halo, dim3(nb_of(nh)), dim3(AHF_BLOCK), 0, st, hout, nh, npart_out, props_out);
   if (ne > 0)
