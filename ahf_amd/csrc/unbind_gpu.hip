@@ -1832,9 +1832,14 @@ __device__ __forceinline__ int64_t group_cut(const UnbindConst &K, int64_t n, co
  * twenty): in the form of its full list the cut members would be carried
  * through every iteration.  A halo that is chunked at any rate makes its cut
  * there (pad: the cut is still to be made).  The record's fields are the
- * cut's, or cleared.  Every form waits for it: 43 us for the 2,437 gathered
- * haloes of a 256^3 box, 57 for 4,000 lists, 238 for 20,000 (random reads of
- * records, most of them beyond the cut: so the step of 256 members first).
+ * cut's, or cleared.
+ *
+ * Every form waits for it.  The additions to one counter follow each other at
+ * about 12 ns, so a workgroup keeps the haloes of the one-wavefront forms, the
+ * most of them, and lists them 64 at a time: 20,000 lists 85 us, added one by one
+ * 238; 4,000 lists 41 and 57, 2,437 gathered ones of a 256^3 box 38 and 43.  Large
+ * haloes are listed at once, about in order's order, as their forms wait for
+ * the longest.
  */
 __global__ void __launch_bounds__(AHF_BLOCK) k_bin_forms(UnbindConst K, const int64_t *__restrict__ off,
                                                   const int32_t *__restrict__ order, int64_t q0, int64_t nh,
@@ -1843,6 +1848,21 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_bin_forms(UnbindConst K, const in
                                                   int32_t *__restrict__ list, int32_t *__restrict__ cnt,
                                                   HaloOut *__restrict__ out)
 {
+  /* the haloes kept, one a lane of the first wavefront */
+  int held = 0, kept_h = 0, kept_f = 0;
+  auto list_kept = [&]() {
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    for (int f = UF_WAVE; f < UF_FORMS; f++) {
+      const uint64_t m = __ballot(lane < held && kept_f == f);
+      if (m == 0ull) continue;
+      const int first = __builtin_ctzll(m);
+      int at = 0;
+      if (lane == first) at = atomicAdd(cnt + f, __popcll(m));
+      at = __shfl(at, first, 64) + __popcll(m & ((1ull << lane) - 1ull));
+      if ((m >> lane) & 1ull) list[f * nh + at] = kept_h;
+    }
+  };
   for (int64_t q = q0 + blockIdx.x; q < nh; q += gridDim.x) {
     const int64_t h = order ? order[q] : q, o = off[h];
     int64_t n = off[h + 1] - o;
@@ -1857,14 +1877,24 @@ __global__ void __launch_bounds__(AHF_BLOCK) k_bin_forms(UnbindConst K, const in
         r.pad = 1;
       }
     }
+    int f = 0;
+    while (f + 1 < UF_FORMS && n < least.v[f]) f++;
     if (threadIdx.x == 0) {
       r.npart = n;
       out[h] = r;
-      int f = 0;
-      while (f + 1 < UF_FORMS && n < least.v[f]) f++;
-      list[f * nh + atomicAdd(cnt + f, 1)] = (int32_t)h;
+      if (f < UF_WAVE) list[f * nh + atomicAdd(cnt + f, 1)] = (int32_t)h;
+    }
+    if (f < UF_WAVE) continue;
+    if ((int)threadIdx.x == held) {
+      kept_h = (int)h;
+      kept_f = f;
+    }
+    if (++held == 64) {
+      list_kept();
+      held = 0;
     }
   }
+  list_kept();
 }
 
 /* plain form: one halo per launch */

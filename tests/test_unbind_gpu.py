@@ -499,6 +499,32 @@ def test_many_short_haloes(oracle, ctx, tmp_path, cuts):
     _compare(ref, npart, props, lists, f"short haloes {cuts}")
 
 
+def test_more_haloes_than_a_workgroup_keeps(oracle, ctx, tmp_path):
+    """more than 64 short haloes for each workgroup that lists them by form,
+    with two larger ones among them"""
+    rng = np.random.default_rng(12)
+    nh = 140000
+    sizes = np.where(rng.random(nh) < 0.9, 20, 24)
+    sizes[[5, 90001]] = 700, 3000
+    n, off = int(sizes.sum()), np.concatenate([[0], np.cumsum(sizes)])
+    cen = np.float32(rng.uniform(0.05, 0.95, (nh, 3))).astype(np.float64)
+    d = rng.standard_normal((n, 3))
+    r = 0.002 * rng.random(n) ** 1.5
+    pos = (np.repeat(cen, sizes, axis=0) + r[:, None] * d / np.linalg.norm(d, axis=1)[:, None]).astype(np.float32)
+    mom = rng.standard_normal((n, 3)) * 0.02
+    mom[rng.random(n) < 0.1] *= 4.0
+    snap, out = str(tmp_path / "k.snap"), str(tmp_path / "o.halo")
+    dumps.write_snapshot(snap, pos, mom, boxsize=1.0, pmass=1e8, L_dom=16, centres=cen,
+                         halo_lists=[np.arange(off[h], off[h + 1], dtype=np.uint64) for h in range(nh)], r_fac=1.0,
+                         v_fac=1.0, phi_fac=2e-7, hubble=10.0, ovlim=200.0, rho_vir=3e14, gather_rad=np.full(nh, 0.004))
+    assert oracle.oracle_construct_dump(snap.encode(), out.encode(), 8, 0) == 0
+    ref = dumps.read_halos(out)
+    s = dumps.read_snapshot(snap)
+    assert np.any(ref.npart == s.halo_npart) and np.any(ref.npart < s.halo_npart)
+    _, (npart, props, lists) = _construct_gpu(ctx, s, WITH_RVIR)
+    _compare(ref, npart, props, lists, "140,000 haloes")
+
+
 def test_schedule_file(tmp_path, monkeypatch):
     """a context applies the schedule file named by AHF_SCHEDULE"""
     import json
