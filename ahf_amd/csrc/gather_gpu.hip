@@ -273,6 +273,7 @@ extern "C" int ahfgpu_gather_halos(ahfgpu_ctx *c, const double *centres, const d
   }
   c->timers_collect();
   c->gather_candidates = nc;
+  s->gathered = 1;
   c->halo_set = s;
   return 0;
 }

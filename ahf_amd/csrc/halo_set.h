@@ -39,6 +39,7 @@ struct HaloSet {
   std::vector<int32_t> h_ord; /* the host copy of order */
   HaloOut *out = nullptr;
   uint32_t *buf_a = nullptr, *buf_b = nullptr;
+  int gathered = 0; /* the lists are the library's own gather's */
   int done = 0;
   int res_staged = 0; /* the results are in `res` already (read back with the unbinding's own synchronisation) */
   char *dev = nullptr, *host = nullptr;
@@ -75,6 +76,7 @@ static inline int halo_set_reserve(ahfgpu_ctx *c, int64_t nh, int64_t ne, HaloSe
   }
   if (!s) s = new HaloSet();
   c->halo_set = nullptr;
+  s->gathered = 0;
   s->done = 0;
   s->res_staged = 0;
   s->out = nullptr;

@@ -3352,8 +3352,8 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     /* the order is largest first: haloes of split_min members or more take
      * the split path on the second stream, the others the forms by size: the
      * wavefront forms on the third stream, the workgroup forms on the first
-     * (which stream the chunked form, 4097 members to split_min, has depends on
-     * the split path: below) */
+     * (where the chunked form, 4097 members to split_min, and the big one run
+     * depends on the split path: below) */
     int64_t nsplit = 0;
     const std::vector<int32_t> &ord = s->h_ord;
     const int64_t split_min = c->split_min > 0 ? c->split_min : AHF_SPLIT_DEFAULT;
@@ -3411,7 +3411,13 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
   } while (0)
     hipStream_t sw = fork ? c->st3 : c->st;
     /* the chunked form has the second stream, or the first where the split
-     * path has that one; the big form is then beside the others on the third */
+     * path has that one; the big form then follows it, or, where its lists take
+     * long, is ahead of the others on the third.  Long are given lists of 8192
+     * members or more; gathered ones keep about one in twenty.  (Unbinding alone,
+     * on the third stream and behind the chunked form: a 256^3 box's gathered
+     * haloes 0.96 and 0.70 ms, its given ones with 7,421 members at most unsplit
+     * 0.60 and 0.57; 20,000 haloes with lists up to the split path's 2.52 and
+     * 2.96.) */
     const bool chunk1 = most(UF_CHUNK) > 0 && nsplit > 0;
     const bool chunk2 = most(UF_CHUNK) > 0 && !chunk1;
     if (chunk2) {
@@ -3423,7 +3429,8 @@ extern "C" int ahfgpu_unbind(ahfgpu_ctx *c, const ahfgpu_unbind_params *p, int m
     /* binned, every form may hold long-running haloes: the middle one on
      * another stream than the big one's, the second if nothing else is there */
     const bool mid2 = binned && fork && nsplit == 0 && most(UF_CHUNK) == 0 && most(UF_BIG) > 0;
-    hipStream_t sb = chunk1 && wvs > 0 ? sw : c->st;
+    const bool long_chunk = chunk1 && !(s->gathered && binned) && size_of(nsplit) >= 8192;
+    hipStream_t sb = long_chunk && wvs > 0 ? sw : c->st;
     hipStream_t sm = mid2 ? c->st2 : (chunk1 || (binned && fork && most(UF_BIG) > 0)) && wvs > 0 ? sw : c->st;
     if (wvs > 0 && fork) hipStreamWaitEvent(sw, c->ev_s0, 0);
     if (mid2) hipStreamWaitEvent(c->st2, c->ev_s0, 0);
