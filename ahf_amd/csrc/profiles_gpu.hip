@@ -2049,6 +2049,9 @@ extern "C" int ahfgpu_halo_profiles(ahfgpu_ctx *c, const ahfgpu_profile_params *
   double *d_props = A.get<double>(nh * PP_N), *d_prof = A.get<double>(tot * PQ_N);
   if (!d_props || !d_prof || (nbig && !d_big)) return c->fail(AHFGPU_ENOMEM, "device arena exhausted (profiles)");
   auto get_rows = [&]() {
+    /* no map, no tiled haloes: k_profiles asks for both by the pointers */
+    d_tl = nullptr;
+    d_tmap = nullptr;
     if (ntl == 0) return true;
     d_tl = A.get<PrfTiled>(ntl);
     d_tile = A.get<PrfTile>(ntile);

@@ -176,28 +176,33 @@ def test_profiles_beside_others(ctx, sizes):
 def test_profiles_without_room(ctx, sizes, fits):
     """haloes below 32768 members do without the rows of the walk over the
     device where there is no room for them, and give the same bits; the larger
-    ones need theirs"""
+    ones need theirs.  The calls without room are a context's first, with
+    nothing of an earlier call in its memory."""
     import ahf_amd
-    centre, ip, pr = _given_haloes(ctx, sizes)
     args = (20, 1.0, 1.0, 1.0, 1.0, 0.1)
+    centre, ip, pr = _given_haloes(ctx, sizes)
     ctx.set_halos(centre, np.array(sizes, np.int64), ip)
     ref = ctx.halo_profiles(*args, phi0_rvir=pr)
+    c = ahf_amd.Context(0)
     try:
+        centre, ip, pr = _given_haloes(c, sizes)
+        c.set_halos(centre, np.array(sizes, np.int64), ip)
         # 24 bytes a member for every call, 164 for each one that has rows; the
         # haloes' records and the tiles' take less than the 400,000 beside them
-        ctx.set_memory_limit(24 * sum(sizes) + 164 * (fits or 0) + 400000)
+        c.set_memory_limit(24 * sum(sizes) + 164 * (fits or 0) + 400000)
         if fits is None:
             with pytest.raises(ahf_amd.AhfGpuError):
-                ctx.halo_profiles(*args, phi0_rvir=pr)
+                c.halo_profiles(*args, phi0_rvir=pr)
         else:
-            _same_profiles(ctx.halo_profiles(*args, phi0_rvir=pr), ref)
-        ctx.set_schedule(prof_tiled=8192)
+            _same_profiles(c.halo_profiles(*args, phi0_rvir=pr), ref)
+        c.set_schedule(prof_tiled=8192)
         with pytest.raises(ahf_amd.AhfGpuError):
-            ctx.halo_profiles(*args, phi0_rvir=pr)
+            c.halo_profiles(*args, phi0_rvir=pr)
+        c.set_memory_limit(0)
+        c.set_schedule(prof_tiled=0)
+        _same_profiles(c.halo_profiles(*args, phi0_rvir=pr), ref)
     finally:
-        ctx.set_memory_limit(0)
-        _reset_split(ctx)
-    _same_profiles(ctx.halo_profiles(*args, phi0_rvir=pr), ref)
+        c.close()
 
 
 @pytest.mark.parametrize("cfg,side,seed,gather", [(2, 800, 1002, 0), (3, 48, 5, 0), (2, 400, 1002, 1)])
